@@ -1,12 +1,10 @@
 // Batched strided split-K GEMM on gfx950 matrix cores.
 //
-// Tile: BM x BN per workgroup of 256 threads (4 wave64s arranged 2x2), each
-// wave owns a (BM/2) x (BN/2) sub-tile made of 16x16 MFMA blocks.  K is staged
-// through LDS in BK=16 slices, double buffered: the next slice is fetched into
-// registers while the matrix cores work on the current one.
-//
-// FP64 path: v_mfma_f64_16x16x4_f64 (one double of A and of B per lane per
-// instruction, 4 doubles of C per lane).
+// FP64: v_mfma_f64_16x16x4_f64 (one double of A and of B per lane per instruction, 4
+// doubles of C per lane) on 64- or 128-row tiles of 16 to 144 columns; described at
+// dgemm_f64_tile, chosen in plan_f64.
+// FP32: BM x BN tiles per workgroup of 256 threads (4 wave64s arranged 2x2), K staged
+// through LDS in BK=16 slices, double buffered; described at sgemm_f32acc64_tile.
 //
 // Operand fragments for a 16x16x4 block (lane l, r = 0..3):
 //   A[m = l%16][k = l/16], B[k = l/16][n = l%16], C[m = 4*r + l/16][n = l%16]
@@ -53,77 +51,161 @@ __device__ inline int xcd_tile(const KParams& p) {
   return t < p.tiles_m * p.tiles_n ? t : -1;
 }
 
-// One BM x BN output tile `tile` (row-major tile index) of batch/split slice z
-// (z = batch * nsplit + split, batch relative to p.batch0).  Called by all 256
-// threads of a workgroup.
-template <int BM, int BN, bool TA, bool TB>
-__device__ __forceinline__ void dgemm_f64_tile(const KParams& p, int tile, int z) {
-  constexpr int PAD = 1;
-  constexpr int LDA_S = BM + PAD;
-  constexpr int LDB_S = BN + PAD;
-  constexpr int A_PER = BM * kBK / kThreads;
-  constexpr int B_PER = BN * kBK / kThreads;
-  constexpr int WM = BM / 2, WN = BN / 2;  // wave sub-tile
-  constexpr int RB = WM / 16, CB = WN / 16;
+// ---------------------------------------------------------------- FP64 tile
+// One 64 RB x 16 CB output tile `tile` (row-major tile index) of batch/split slice z
+// (z = batch * nsplit + split, batch relative to p.batch0), by KG groups of four
+// wave64s.  Bound: the matrix cores, one v_mfma_f64_16x16x4f64 per 64 cycles and SIMD
+// (78.6 TFLOP/s), so everything else has to leave their issue slots alone:
+//  * The four waves of a group are stacked along M (16 RB rows each, all 16 CB columns),
+//    so a row of A belongs to one wave and its fragments go straight from global memory
+//    to registers (whole 128-byte row pieces for A, 128-byte runs of m for A^T), one
+//    K slice of 16 U values (U = 2 for small tiles) ahead of the products.  Only B, shared by the waves, is staged
+//    through LDS (double buffered, one barrier per slice), in 16-byte pieces.
+//  * No bounds check in the K loop: rows and columns past the edge read clamped
+//    addresses, and the last, partial K slice goes through checked loads with zeros.
+//  * CB (1 .. 9) follows N, so that o^2, o v, nbf ... wide outputs are not padded to 64.
+//  * KG groups split K inside the workgroup (their sums are added through LDS in group
+//    order), for outputs of too few tiles to give every SIMD two waves.
+// Measured in TFLOP/s (before: 2 x 2 waves, both operands through LDS in checked 8-byte loads,
+// 64 or 128 columns): 65536 x 1024 x 65536 58.6 -> 69.8 (the rate of a large library product here: 70 to 72), 3420^3 51.5 ->
+// 63.6, 6555 x 900 x 6555 46.7 -> 62.0, 1520^3 42.5 -> 55.2, 2985984 x 144 x 144 (A^T) 35.9 ->
+// 52.9, 900^3 28.3 -> 37.7; 95^3 8.9 -> 5.5 us.  Tried and dropped: exec-masked loads
+// in place of clamped ones (the wait for a masked load moves up to where it merges with the
+// unloaded value: 1520^3 55 -> 49), slices of 32 for the large tiles (no gain).
+// A slice's k = 16 t + 4 (lane / 16) + q belongs to the q-th of its four MFMA steps (any
+// assignment is exact when A and B use the same one).
+typedef double double2a8 __attribute__((ext_vector_type(2), aligned(8)));  // 16-byte load at 8-byte alignment
 
-  __shared__ double As[2][kBK][LDA_S];
-  __shared__ double Bs[2][kBK][LDB_S];
+template <int CB, int U, bool TB>
+struct F64Lds {
+  static constexpr int kSlice = 16 * U;
+  // pitches that keep the fragment reads off each other's banks
+  static constexpr int kPitch = TB ? kSlice + 2 : 16 * CB + 4;
+  static constexpr int kRows = TB ? 16 * CB : kSlice;
+  static constexpr int kDoubles = kRows * kPitch;
+};
 
-  const int tid = threadIdx.x;
+template <int RB, int CB, int KG, int U, bool TA, bool TB>
+struct F64Shared {
+  static constexpr int kStage = 2 * KG * F64Lds<CB, U, TB>::kDoubles;
+  static constexpr int kReduce = KG > 1 ? 64 * RB * 16 * CB : 0;
+  static constexpr int kDoubles = kStage > kReduce ? kStage : kReduce;
+};
+
+template <int RB, int CB, int KG, int U, bool TA, bool TB>
+__device__ __forceinline__ void dgemm_f64_tile(const KParams& p, int tile, int z, double* __restrict__ smem) {
+  constexpr int BM = 64 * RB, BN = 16 * CB, BK = 16 * U;
+  constexpr int PITCH = F64Lds<CB, U, TB>::kPitch;
+
+  const int tid = threadIdx.x & (kThreads - 1);
+  const int grp = KG > 1 ? __builtin_amdgcn_readfirstlane(threadIdx.x / kThreads) : 0;
+  double* const Bs = smem + grp * 2 * F64Lds<CB, U, TB>::kDoubles;
   const int lane = tid & 63;
   const int wave = tid >> 6;
-  const int wm = wave >> 1, wn = wave & 1;
   const int lr = lane & 15, lk = lane >> 4;
 
   const int tm = tile / p.tiles_n, tn = tile - tm * p.tiles_n;
   const int b = p.batch0 + z / p.nsplit;
   const int s = z - (z / p.nsplit) * p.nsplit;
   const int m0 = tm * BM, n0 = tn * BN;
-  const int k_begin = s * p.kchunk;
-  const int k_end = min(p.K, k_begin + p.kchunk);
+  int k_begin = s * p.kchunk;
+  int k_end = min(p.K, k_begin + p.kchunk);
+  int nslices = (k_end - k_begin + BK - 1) / BK;               // of the longest group
+  if (KG > 1) {
+    const int per = (nslices + KG - 1) / KG;
+    k_begin += grp * per * BK;
+    k_end = min(k_end, k_begin + per * BK);
+    nslices = per;
+  }
+  const int full = k_end > k_begin ? (k_end - k_begin) / BK : 0;  // whole slices of this group
 
-  const double* __restrict__ A = p.A + (long)b * p.sA;
-  const double* __restrict__ B = p.B + (long)b * p.sB;
-
-  double ra[A_PER], rb[B_PER];
-
-  auto load_regs = [&](int k0) {
+  // Every load of a whole slice is unconditional (a masked one would be waited for where
+  // its register merges with the unloaded value): rows and columns past the edge read the
+  // last ones instead, and their products are never stored.
+  // A: this lane's row of each 16-row block.
+  const double* ap[RB];
 #pragma unroll
-    for (int r = 0; r < A_PER; ++r) {
-      const int e = tid + kThreads * r;
-      int mm, kk;
-      if (!TA) { mm = e / kBK; kk = e % kBK; } else { kk = e / BM; mm = e % BM; }
-      const int gm = m0 + mm, gk = k0 + kk;
-      double x = 0.0;
-      if (gm < p.M && gk < k_end) x = TA ? A[(long)gk * p.lda + gm] : A[(long)gm * p.lda + gk];
-      ra[r] = x;
+  for (int i = 0; i < RB; ++i) {
+    const long m = min(m0 + (wave * RB + i) * 16 + lr, p.M - 1);
+    ap[i] = p.A + (long)b * p.sA + (TA ? (long)(k_begin + 4 * lk) * p.lda + m : m * p.lda + k_begin + 4 * lk);
+  }
+  // B: this thread's 16-byte pieces, kStep columns (rows, for B^T) apart.  With an odd N
+  // the pair of the last column starts one earlier and is put right when it is stored.
+  constexpr int kLine = TB ? BK / 2 : kThreads / BK;  // threads per row of the stage
+  constexpr int kStep = TB ? kThreads / kLine : 2 * kLine;
+  constexpr int PER = (BN + kStep - 1) / kStep;
+  const int bk = TB ? 2 * (tid % kLine) : tid / kLine;   // first k of the pieces
+  const int bn0 = TB ? tid / kLine : 2 * (tid % kLine);  // n of piece 0
+  const double* bp = p.B + (long)b * p.sB + (TB ? (long)(k_begin + bk) : (long)(k_begin + bk) * p.ldb);
+  long boff[PER];
+#pragma unroll
+  for (int r = 0; r < PER; ++r) {
+    const int n = n0 + bn0 + kStep * r;
+    boff[r] = TB ? (long)min(n, p.N - 1) * p.ldb : (long)max(0, min(n, p.N - 2));
+  }
+  double* const bdst = Bs + (TB ? bn0 * PITCH + bk : bk * PITCH + bn0);
+  const bool odd_edge = !TB && (p.N & 1) && n0 + BN >= p.N;  // some thread has half a piece
+  const bool narrow = !TB && p.N < 2;                        // no whole piece in a row of B
+
+  double an[RB][4 * U];  // next slice's fragments of A
+  double2a8 bn[PER];     // next slice's pieces of B
+  auto load_full = [&]() {
+#pragma unroll
+    for (int i = 0; i < RB; ++i) {
+      if (TA) {
+#pragma unroll
+        for (int q = 0; q < 4 * U; ++q) an[i][q] = ap[i][(long)(16 * (q / 4) + q % 4) * p.lda];
+      } else {
+#pragma unroll
+        for (int q = 0; q < 4 * U; q += 2) {
+          const double2a8 x = *reinterpret_cast<const double2a8*>(ap[i] + 16 * (q / 4) + q % 4);
+          an[i][q] = x[0];
+          an[i][q + 1] = x[1];
+        }
+      }
+      ap[i] += TA ? (long)BK * p.lda : BK;
     }
 #pragma unroll
-    for (int r = 0; r < B_PER; ++r) {
-      const int e = tid + kThreads * r;
-      int nn, kk;
-      if (!TB) { kk = e / BN; nn = e % BN; } else { nn = e / kBK; kk = e % kBK; }
-      const int gn = n0 + nn, gk = k0 + kk;
-      double x = 0.0;
-      if (gn < p.N && gk < k_end) x = TB ? B[(long)gn * p.ldb + gk] : B[(long)gk * p.ldb + gn];
-      rb[r] = x;
-    }
+    for (int r = 0; r < PER; ++r) bn[r] = *reinterpret_cast<const double2a8*>(bp + boff[r]);
+    bp += TB ? BK : (long)BK * p.ldb;
   };
-  auto store_lds = [&](int buf) {
+  // a slice that K ends in (or any slice of a one-column B), element by element: zeros
+  // from k_end on
+  auto load_checked = [&](int t) {
+    const int k0 = k_begin + t * BK;
 #pragma unroll
-    for (int r = 0; r < A_PER; ++r) {
-      const int e = tid + kThreads * r;
-      int mm, kk;
-      if (!TA) { mm = e / kBK; kk = e % kBK; } else { kk = e / BM; mm = e % BM; }
-      As[buf][kk][mm] = ra[r];
+    for (int i = 0; i < RB; ++i) {
+#pragma unroll
+      for (int q = 0; q < 4 * U; ++q) {
+        const int dk = 16 * (q / 4) + q % 4;
+        an[i][q] = k0 + 4 * lk + dk < k_end ? ap[i][TA ? (long)dk * p.lda : dk] : 0.0;
+      }
+      if (narrow) ap[i] += TA ? (long)BK * p.lda : BK;
     }
 #pragma unroll
-    for (int r = 0; r < B_PER; ++r) {
-      const int e = tid + kThreads * r;
-      int nn, kk;
-      if (!TB) { kk = e / BN; nn = e % BN; } else { nn = e / kBK; kk = e % kBK; }
-      Bs[buf][kk][nn] = rb[r];
+    for (int r = 0; r < PER; ++r)
+#pragma unroll
+      for (int h = 0; h < 2; ++h) {
+        const int k = k0 + bk + (TB ? h : 0);
+        bn[r][h] = k < k_end ? bp[boff[r] + (narrow ? 0 : h)] : 0.0;
+      }
+    if (narrow) bp += (long)BK * p.ldb;
+  };
+  auto load = [&](int t) {
+    if (t < full && !narrow) load_full();
+    else load_checked(t);
+  };
+  auto store_b = [&](int buf) {
+    if (odd_edge) {
+#pragma unroll
+      for (int r = 0; r < PER; ++r)
+        if (n0 + bn0 + kStep * r == p.N - 1) bn[r][0] = bn[r][1];
     }
+#pragma unroll
+    for (int r = 0; r < PER; ++r)
+      if (BN % kStep == 0 || bn0 + kStep * r < BN)
+        *reinterpret_cast<double2*>(bdst + buf * F64Lds<CB, U, TB>::kDoubles + (TB ? kStep * r * PITCH : kStep * r)) =
+            double2{bn[r][0], bn[r][1]};
   };
 
   double4_t acc[RB][CB];
@@ -132,71 +214,133 @@ __device__ __forceinline__ void dgemm_f64_tile(const KParams& p, int tile, int z
 #pragma unroll
     for (int j = 0; j < CB; ++j) acc[i][j] = double4_t{0.0, 0.0, 0.0, 0.0};
 
-  int buf = 0;
-  if (k_begin < k_end) {
-    load_regs(k_begin);
-    store_lds(0);
-  }
-  __syncthreads();
-  for (int kt = k_begin; kt < k_end; kt += kBK) {
-    const bool has_next = kt + kBK < k_end;
-    if (has_next) load_regs(kt + kBK);
+  // Steps of one slice: one k per lane group for B rows of n, a pair for B rows of k.
+  // The B fragments of a step are read one step ahead of their products, across the
+  // slice's barrier too, which stands before the last step: every wave then has the
+  // slice's last fragments in registers, so its stage is free, and the other stage is
+  // complete.  No product waits for the LDS or, at the barrier, for a slower wave's reads.
+  constexpr int PAIR = TB ? 2 : 1, STEPS = 4 * U / PAIR;
+  auto read_b = [&](int buf, int step, double (&f)[CB][PAIR]) {
+    const double* bs = Bs + buf * F64Lds<CB, U, TB>::kDoubles;
+    if constexpr (TB) {
+      bs += lr * PITCH + 4 * lk + 16 * (step / 2) + 2 * (step % 2);
 #pragma unroll
-    for (int ks = 0; ks < kBK / 4; ++ks) {
-      double fa[RB], fb[CB];
+      for (int j = 0; j < CB; ++j) {
+        const double2 x = *reinterpret_cast<const double2*>(bs + 16 * j * PITCH);
+        f[j][0] = x.x;
+        f[j][PAIR - 1] = x.y;
+      }
+    } else {
+      bs += (4 * lk + 16 * (step / 4) + step % 4) * PITCH + lr;
 #pragma unroll
-      for (int i = 0; i < RB; ++i) fa[i] = As[buf][ks * 4 + lk][wm * WM + i * 16 + lr];
+      for (int j = 0; j < CB; ++j) f[j][0] = bs[16 * j];
+    }
+  };
+  // (the widest tile has no registers left for a second set: it reads a step's fragments
+  // just before the products)
+  constexpr bool kAhead = RB * CB < 18;
+  double a[RB][4 * U], fb[kAhead ? 2 : 1][CB][PAIR];
+  auto products = [&](int step) {
 #pragma unroll
-      for (int j = 0; j < CB; ++j) fb[j] = Bs[buf][ks * 4 + lk][wn * WN + j * 16 + lr];
+    for (int h = 0; h < PAIR; ++h)
 #pragma unroll
       for (int i = 0; i < RB; ++i)
 #pragma unroll
         for (int j = 0; j < CB; ++j)
-          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(fa[i], fb[j], acc[i][j], 0, 0, 0);
+          acc[i][j] = __builtin_amdgcn_mfma_f64_16x16x4f64(a[i][step * PAIR + h], fb[kAhead ? step & 1 : 0][j][h], acc[i][j], 0, 0, 0);
+  };
+  if (nslices > 0) {
+    load(0);
+    store_b(0);
+  }
+  __syncthreads();
+  if (nslices > 0) {
+    if (kAhead) read_b(0, 0, fb[0]);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int q = 0; q < 4 * U; ++q) a[i][q] = an[i][q];
+  }
+  int buf = 0;
+  for (int t = 0; t < nslices; ++t) {
+    const bool has_next = t + 1 < nslices;
+    if (has_next) load(t + 1);
+#pragma unroll
+    for (int step = 0; step < STEPS - 1; ++step) {
+      if constexpr (kAhead) {
+        read_b(buf, step + 1, fb[(step + 1) & 1]);
+        __builtin_amdgcn_sched_barrier(0);  // the reads stay ahead of the products
+      } else {
+        read_b(buf, step, fb[0]);
+      }
+      products(step);
     }
-    if (has_next) store_lds(buf ^ 1);
+    if (!kAhead) read_b(buf, STEPS - 1, fb[0]);
+    if (has_next) store_b(buf ^ 1);
     __syncthreads();
     buf ^= 1;
+    if (kAhead && has_next) read_b(buf, 0, fb[0]);
+    __builtin_amdgcn_sched_barrier(0);
+    products(STEPS - 1);
+#pragma unroll
+    for (int i = 0; i < RB; ++i)
+#pragma unroll
+      for (int q = 0; q < 4 * U; ++q) a[i][q] = an[i][q];
+  }
+  if (KG > 1) __syncthreads();
+
+  if (KG > 1) {  // (every wave has left the K loop: the stages are free)
+#pragma unroll 1
+    for (int g = 1; g < KG; ++g) {
+      if (grp == g) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+          for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) smem[((i * CB + j) * 4 + r) * kThreads + tid] = acc[i][j][r];
+      }
+      __syncthreads();
+      if (grp == 0) {
+#pragma unroll
+        for (int i = 0; i < RB; ++i)
+#pragma unroll
+          for (int j = 0; j < CB; ++j)
+#pragma unroll
+            for (int r = 0; r < 4; ++r) acc[i][j][r] += smem[((i * CB + j) * 4 + r) * kThreads + tid];
+      }
+      __syncthreads();
+    }
+    if (grp != 0) return;
   }
 
-  // epilogue
-  if (p.nsplit == 1) {
-    double* __restrict__ C = p.C + (long)b * p.sC;
+  // epilogue: C, or partial sums to workspace slice z (dense M x N)
+  const bool split = p.nsplit > 1;
+  double* __restrict__ out = split ? p.W + (long)z * p.M * p.N : p.C + (long)b * p.sC;
+  const long ldo = split ? p.N : p.ldc;
+  const double beta = split ? 0.0 : p.beta;
 #pragma unroll
-    for (int i = 0; i < RB; ++i)
+  for (int i = 0; i < RB; ++i)
 #pragma unroll
-      for (int j = 0; j < CB; ++j)
+    for (int r = 0; r < 4; ++r) {
+      const int gm = m0 + (wave * RB + i) * 16 + r * 4 + lk;
+      if (gm >= p.M) continue;
+      double* c = out + (long)gm * ldo + n0 + lr;
 #pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gm = m0 + wm * WM + i * 16 + r * 4 + lk;
-          const int gn = n0 + wn * WN + j * 16 + lr;
-          if (gm < p.M && gn < p.N) {
-            double* c = C + (long)gm * p.ldc + gn;
-            const double v = p.alpha * acc[i][j][r];
-            *c = (p.beta == 0.0) ? v : v + p.beta * (*c);
-          }
-        }
-  } else {
-    // partial sums to workspace slice z (dense M x N)
-    double* __restrict__ Wz = p.W + (long)z * p.M * p.N;
-#pragma unroll
-    for (int i = 0; i < RB; ++i)
-#pragma unroll
-      for (int j = 0; j < CB; ++j)
-#pragma unroll
-        for (int r = 0; r < 4; ++r) {
-          const int gm = m0 + wm * WM + i * 16 + r * 4 + lk;
-          const int gn = n0 + wn * WN + j * 16 + lr;
-          if (gm < p.M && gn < p.N) Wz[(long)gm * p.N + gn] = p.alpha * acc[i][j][r];
-        }
-  }
+      for (int j = 0; j < CB; ++j) {
+        if (n0 + 16 * j + lr >= p.N) continue;
+        const double v = p.alpha * acc[i][j][r];
+        c[16 * j] = (beta == 0.0) ? v : v + beta * c[16 * j];
+      }
+    }
 }
 
-template <int BM, int BN, bool TA, bool TB>
-__global__ __launch_bounds__(kThreads, 2) void dgemm_f64_kernel(KParams p) {
+template <int RB, int CB, int KG, int U, bool TA, bool TB>
+__global__ __launch_bounds__(kThreads * KG, KG > 2 ? KG : 2) void dgemm_f64_kernel(KParams p) {
+  __shared__ __attribute__((aligned(16))) double smem[F64Shared<RB, CB, KG, U, TA, TB>::kDoubles];
   const int tile = xcd_tile(p);
   if (tile < 0) return;
-  dgemm_f64_tile<BM, BN, TA, TB>(p, tile, blockIdx.y);
+  dgemm_f64_tile<RB, CB, KG, U, TA, TB>(p, tile, blockIdx.y, smem);
 }
 
 // FP32 path: operands are rounded to FP32 when staged into LDS and multiplied
@@ -483,7 +627,7 @@ bool wide_tiles(const GemmDesc& d, size_t ws_bytes) {
 }
 
 template <int BM, int BN>
-void launch(const GemmDesc& d, GemmPrecision prec, const GemmWorkspace& ws, hipStream_t stream) {
+void launch_f32(const GemmDesc& d, const GemmWorkspace& ws, hipStream_t stream) {
   const int tiles_m = (int)ceil_div(d.M, BM), tiles_n = (int)ceil_div(d.N, BN);
   const long tiles = (long)tiles_m * tiles_n;
   const SplitKPlan plan = plan_splitk(d, BM, BN, ws.bytes);
@@ -497,20 +641,124 @@ void launch(const GemmDesc& d, GemmPrecision prec, const GemmWorkspace& ws, hipS
     p.tiles_m = tiles_m; p.tiles_n = tiles_n; p.alpha = d.alpha; p.beta = d.beta;
     p.per_xcd = tiles >= kXcdMinTiles ? (int)ceil_div(tiles, kXcdCount) : 0;
     dim3 grid((unsigned)(p.per_xcd ? p.per_xcd * kXcdCount : tiles), (unsigned)(nb * nsplit));
-    if (prec == GemmPrecision::F32) {
-      if (!d.transA && !d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, false, false>), grid, dim3(kThreads), 0, stream, p);
-      else if (!d.transA && d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, false, true>), grid, dim3(kThreads), 0, stream, p);
-      else if (d.transA && !d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, true, false>), grid, dim3(kThreads), 0, stream, p);
-      else hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, true, true>), grid, dim3(kThreads), 0, stream, p);
-      check_launch("sgemm_f32acc64");
-    } else {
-      if (!d.transA && !d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<BM, BN, false, false>), grid, dim3(kThreads), 0, stream, p);
-      else if (!d.transA && d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<BM, BN, false, true>), grid, dim3(kThreads), 0, stream, p);
-      else if (d.transA && !d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<BM, BN, true, false>), grid, dim3(kThreads), 0, stream, p);
-      else hipLaunchKernelGGL((dgemm_f64_kernel<BM, BN, true, true>), grid, dim3(kThreads), 0, stream, p);
-      check_launch("dgemm_f64");
-    }
+    if (!d.transA && !d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, false, false>), grid, dim3(kThreads), 0, stream, p);
+    else if (!d.transA && d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, false, true>), grid, dim3(kThreads), 0, stream, p);
+    else if (d.transA && !d.transB) hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, true, false>), grid, dim3(kThreads), 0, stream, p);
+    else hipLaunchKernelGGL((sgemm_f32acc64_kernel<BM, BN, true, true>), grid, dim3(kThreads), 0, stream, p);
+    check_launch("sgemm_f32acc64");
     if (nsplit > 1) splitk_reduce(ws.ptr, d.C, d.ldc, d.sC, d.M, d.N, nsplit, b0, nb, d.beta, stream);
+  }
+}
+
+// ---------------------------------------------------------------- FP64 plan
+// Tile, K groups and K splits of an FP64 contraction, chosen by a time model in cycles of
+// a SIMD.  Its constants were fitted to 2,000 timings (every tile with one to three
+// workgroups per CU on 60 shapes of M, N from 1 to 3e6 and K from 7 to 4e5): the choice
+// is within 1.5 % of the fastest tile on average, and within 11 %.  In it
+//  * the busiest CU runs its workgroups `occ` at a time, and each lot takes the longer of
+//    its products (64 cycles each, 4 u rb cb per slice and SIMD) and a lone group's time
+//    (its slices, each at least a load's latency, the prologue, the sums over groups);
+//  * operand rows reach the CUs at 3.6 KB and HBM delivers 2.1 KB per cycle;
+//  * a K split costs a launch and its partials' way through HBM.
+// tile: 64 rb x 16 cb outputs, kg groups, slices of 16 u values of k; occ: workgroups per CU
+#define MPQC_F64_TILES(X)                                                                          \
+  X(2, 9, 1, 1, 2) X(2, 8, 1, 1, 2) X(2, 7, 1, 1, 2) X(2, 6, 1, 1, 2) X(2, 5, 1, 1, 2)             \
+  X(2, 4, 1, 1, 3) X(2, 3, 1, 2, 2) X(1, 9, 1, 1, 2) X(1, 8, 1, 1, 2) X(1, 6, 1, 2, 3)             \
+  X(1, 5, 1, 2, 3) X(1, 4, 1, 2, 3) X(1, 5, 2, 2, 1) X(1, 4, 2, 2, 1) X(1, 3, 2, 2, 1)             \
+  X(1, 2, 2, 2, 2) X(1, 4, 4, 1, 1) X(1, 3, 4, 1, 1) X(1, 2, 4, 1, 1) X(1, 2, 4, 2, 1)             \
+  X(1, 1, 4, 2, 1)
+struct F64Tile { int rb, cb, kg, u, occ; };
+constexpr F64Tile kF64Tiles[] = {
+#define X(RB, CB, KG, U, OCC) {RB, CB, KG, U, OCC},
+    MPQC_F64_TILES(X)
+#undef X
+};
+constexpr int kF64TileCount = (int)(sizeof(kF64Tiles) / sizeof(kF64Tiles[0]));
+
+struct F64Plan {
+  int tile = 0;  // of kF64Tiles
+  int nsplit = 1, kchunk = 0, max_batch_per_launch = 65535;
+  size_t scratch_bytes = 0;
+};
+
+constexpr int kCUs = 256;
+
+F64Plan plan_f64(const GemmDesc& d, size_t ws_bytes) {
+  const size_t slice_bytes = (size_t)d.M * d.N * sizeof(double);
+  const double hbm = ((double)d.M * d.K + (double)d.K * d.N + (double)d.M * d.N) * d.batch * 8.0 / 2100.0;
+  F64Plan best;
+  double best_t = -1.0;
+  for (int ti = 0; ti < kF64TileCount; ++ti) {
+    const F64Tile& c = kF64Tiles[ti];
+    const long slices = ceil_div(d.K, 16 * c.u);
+    const long work = ceil_div(d.M, 64 * c.rb) * ceil_div(d.N, 16 * c.cb) * d.batch;
+    const double own = c.rb * c.cb * c.u * 256.0;  // products of a slice, per SIMD
+    // splits that give each CU up to three workgroups, at least 128 values of k long
+    long last = 0;
+    for (int want = 1; want <= 3; ++want) {
+      long ns = std::max<long>(1, std::min<long>(std::min<long>(512, d.K / 128), (long)want * kCUs / work));
+      if (ns > 1) ns = std::max<long>(1, std::min<long>(ns, (long)(ws_bytes / slice_bytes)));
+      const long chunk = ceil_div(slices, ns);
+      ns = ceil_div(slices, chunk);
+      if (ns == last) continue;
+      last = ns;
+      const long n = ceil_div(work * ns, kCUs);  // workgroups of the busiest CU
+      const double one = chunk * own * 1.11 + 2200.0;
+      const double lone = ceil_div(chunk, c.kg) * std::max(own + 1250.0, 1900.0) + 2800.0 + (c.kg - 1) * c.rb * c.cb * 1170.0;
+      double t = (double)(n / c.occ) * std::max(c.occ * one, lone);
+      if (n % c.occ) t += std::max((n % c.occ) * one, lone);
+      t = std::max(t, (double)work * ns * chunk * (64 * c.rb + 16 * c.cb) * c.u * 128.0 / 3600.0);
+      t = std::max(t, hbm);
+      if (ns > 1) t += 7400.0 + (double)ns * slice_bytes * d.batch * 2.0 / 2400.0;
+      if (best_t < 0.0 || t < best_t) {
+        best_t = t;
+        best.tile = ti;
+        best.nsplit = (int)ns;
+        best.kchunk = (int)(chunk * 16 * c.u);
+      }
+    }
+  }
+  best.max_batch_per_launch = 65535 / best.nsplit;
+  if (best.nsplit > 1)
+    best.max_batch_per_launch = (int)std::max<size_t>(1, std::min<size_t>(best.max_batch_per_launch,
+                                                                          ws_bytes / (slice_bytes * best.nsplit)));
+  best.scratch_bytes =
+      best.nsplit > 1 ? slice_bytes * best.nsplit * (size_t)std::min(d.batch, best.max_batch_per_launch) : 0;
+  return best;
+}
+
+template <int RB, int CB, int KG, int U>
+void launch_f64_tile(const GemmDesc& d, dim3 grid, const KParams& p, hipStream_t stream) {
+  const dim3 block(kThreads * KG);
+  if (!d.transA && !d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<RB, CB, KG, U, false, false>), grid, block, 0, stream, p);
+  else if (!d.transA && d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<RB, CB, KG, U, false, true>), grid, block, 0, stream, p);
+  else if (d.transA && !d.transB) hipLaunchKernelGGL((dgemm_f64_kernel<RB, CB, KG, U, true, false>), grid, block, 0, stream, p);
+  else hipLaunchKernelGGL((dgemm_f64_kernel<RB, CB, KG, U, true, true>), grid, block, 0, stream, p);
+}
+
+void launch_f64(const GemmDesc& d, const GemmWorkspace& ws, hipStream_t stream) {
+  using Launch = void (*)(const GemmDesc&, dim3, const KParams&, hipStream_t);
+  static constexpr Launch kLaunch[] = {
+#define X(RB, CB, KG, U, OCC) launch_f64_tile<RB, CB, KG, U>,
+      MPQC_F64_TILES(X)
+#undef X
+  };
+  const F64Plan pl = plan_f64(d, ws.bytes);
+  const F64Tile& c = kF64Tiles[pl.tile];
+  const int tiles_m = (int)ceil_div(d.M, 64 * c.rb), tiles_n = (int)ceil_div(d.N, 16 * c.cb);
+  const long tiles = (long)tiles_m * tiles_n;
+  for (int b0 = 0; b0 < d.batch; b0 += pl.max_batch_per_launch) {
+    const int nb = std::min(pl.max_batch_per_launch, d.batch - b0);
+    KParams p;
+    p.A = d.A; p.B = d.B; p.C = d.C; p.W = ws.ptr;
+    p.lda = d.lda; p.ldb = d.ldb; p.ldc = d.ldc; p.sA = d.sA; p.sB = d.sB; p.sC = d.sC;
+    p.M = d.M; p.N = d.N; p.K = d.K; p.kchunk = pl.kchunk; p.nsplit = pl.nsplit; p.batch0 = b0;
+    p.tiles_m = tiles_m; p.tiles_n = tiles_n; p.alpha = d.alpha; p.beta = d.beta;
+    p.per_xcd = tiles >= kXcdMinTiles ? (int)ceil_div(tiles, kXcdCount) : 0;
+    const dim3 grid((unsigned)(p.per_xcd ? p.per_xcd * kXcdCount : tiles), (unsigned)(nb * pl.nsplit));
+    kLaunch[pl.tile](d, grid, p, stream);
+    check_launch("dgemm_f64");
+    if (pl.nsplit > 1) splitk_reduce(ws.ptr, d.C, d.ldc, d.sC, d.M, d.N, pl.nsplit, b0, nb, d.beta, stream);
   }
 }
 
@@ -541,8 +789,12 @@ __global__ __launch_bounds__(kThreads, 2) void grouped_gemm_kernel(const GProble
     const int ntiles = p.tiles_m * p.tiles_n;
     const int z = (int)(local / ntiles);
     const int tile = (int)(local - (long)z * ntiles);
-    if (F32) sgemm_f32acc64_tile<BM, BN, TA, TB>(p, tile, z);
-    else dgemm_f64_tile<BM, BN, TA, TB>(p, tile, z);
+    if constexpr (F32) {
+      sgemm_f32acc64_tile<BM, BN, TA, TB>(p, tile, z);
+    } else {
+      __shared__ __attribute__((aligned(16))) double smem[F64Shared<BM / 64, BN / 16, 1, 1, TA, TB>::kDoubles];
+      dgemm_f64_tile<BM / 64, BN / 16, 1, 1, TA, TB>(p, tile, z, smem);
+    }
     __syncthreads();  // the next item reuses the LDS tiles
   }
 }
@@ -1282,10 +1534,12 @@ void gemm(const GemmDesc& d, GemmPrecision prec, const GemmWorkspace& ws, hipStr
     launch_gemv(d, stream);
     return;
   }
-  if (wide_tiles(d, ws.bytes))
-    launch<128, 128>(d, prec, ws, stream);
+  if (prec == GemmPrecision::F64)
+    launch_f64(d, ws, stream);
+  else if (wide_tiles(d, ws.bytes))
+    launch_f32<128, 128>(d, ws, stream);
   else
-    launch<64, 64>(d, prec, ws, stream);
+    launch_f32<64, 64>(d, ws, stream);
 }
 
 size_t gemm_scratch_bytes(const GemmDesc& d, GemmPrecision prec, size_t ws_bytes) {
@@ -1295,6 +1549,7 @@ size_t gemm_scratch_bytes(const GemmDesc& d, GemmPrecision prec, size_t ws_bytes
   if (!g_thin_k_never && prec == GemmPrecision::F64 &&
       (thin_k_shape(d) || thin_n_shape(d) || small_batched_shape(d) || gemv_shape(d)))
     return 0;
+  if (prec == GemmPrecision::F64) return plan_f64(d, ws_bytes).scratch_bytes;
   const bool wide = wide_tiles(d, ws_bytes);
   return plan_splitk(d, wide ? 128 : 64, wide ? 128 : 64, ws_bytes).scratch_bytes;
 }

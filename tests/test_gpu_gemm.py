@@ -232,3 +232,35 @@ def test_gemm_split_error_bound(prec, ta, tb, m, n, k):
     err = np.abs(dC.cpu().numpy() - ref)
     assert np.all(err <= bound), float((err / bound).max())
     assert err.max() > 1e-15 * np.abs(ref).max()
+
+
+# FP64 tile kernel: one size per tile of the planner (64 or 128 rows, 16 to 144 columns, one
+# to four K groups), odd N (the last 16-byte piece of a row of B), N of 1, K that ends inside
+# a slice, fewer slices than K groups, and K splits.
+@pytest.mark.parametrize("beta", [0.0, -0.3])
+@pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
+@pytest.mark.parametrize("m,n,k,batch", [(63, 1, 40, 3), (65, 15, 95, 1), (95, 95, 31, 1), (361, 25, 361, 1), (90, 90, 9000, 1),
+                                         (129, 143, 600, 1), (1891, 169, 200, 1), (777, 333, 111, 2), (3001, 145, 97, 1),
+                                         (2003, 801, 65, 1), (1000, 1001, 130, 1), (40, 2047, 77, 1)])
+def test_gemm_f64_tiles(ta, tb, m, n, k, batch, beta):
+    from mpqc_amd.ccsd import gemm
+    rng = np.random.default_rng(m + 2 * n + 3 * k)
+    lda, ldb, ldc = (m if ta else k) + 1, (k if tb else n) + (n % 2), n + 3
+    A = rng.standard_normal((batch, k if ta else m, lda))
+    B = rng.standard_normal((batch, n if tb else k, ldb))
+    C = rng.standard_normal((batch, m, ldc))
+    if beta == 0.0:
+        C[:, :, :n] = np.nan
+    a = A[:, :, :m].transpose(0, 2, 1) if ta else A[:, :, :k]
+    b = B[:, :, :k].transpose(0, 2, 1) if tb else B[:, :, :n]
+    ref = C.copy()
+    ref[:, :, :n] = 0.7 * (a @ b) + (beta * C[:, :, :n] if beta != 0.0 else 0.0)
+    dA, dB, dC = _dev(A), _dev(B), _dev(C)
+    gemm(ta, tb, m, n, k, 0.7, dA.data_ptr(), lda, dB.data_ptr(), ldb, beta, dC.data_ptr(), ldc,
+         stride_a=A[0].size, stride_b=B[0].size, stride_c=C[0].size, batch=batch)
+    torch.cuda.synchronize()
+    got = dC.cpu().numpy()
+    assert np.array_equal(got[:, :, n:], C[:, :, n:])  # padding columns untouched
+    # each of k products and sums rounds once in either result: 2 k eps |A| |B|, and the scaling
+    bound = 2 * (k + 4) * 2.3e-16 * (0.7 * (np.abs(a) @ np.abs(b)) + (abs(beta) * np.abs(C[:, :, :n]) if beta else 0.0))
+    assert np.all(np.abs(got[:, :, :n] - ref[:, :, :n]) <= bound)

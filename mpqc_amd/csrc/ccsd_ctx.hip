@@ -716,10 +716,10 @@ PlaneKind CCSDContext::plane_kind() const {
   }
 }
 
-void CCSDContext::ensure_planes(Planes& P, long n) {
-  if (P.p[0] && P.n >= n) return;
+void CCSDContext::ensure_planes(Planes& P, long n, long row) {
+  if (P.p[0] && P.n >= (row ? n / row * plane_pitch(row) : n)) return;
   if (P.p[0]) throw std::logic_error("plane buffer re-sized without release_planes()");
-  P = alloc_planes(n);
+  P = alloc_planes(n, row);
 }
 
 // frees every 16-bit plane buffer and forgets every Planes handle that pointed into them
@@ -736,14 +736,20 @@ void CCSDContext::release_planes() {
   planes_ready_ = false;
 }
 
-Planes CCSDContext::alloc_planes(long n) {
+Planes CCSDContext::alloc_planes(long n, long row) {
   Planes P;
+  if (row && plane_pitch(row) != row) {
+    P.row = row;
+    P.pitch = plane_pitch(row);
+  }
+  n = P.at(n);
   P.n = n;
   for (int q = 0; q < plane_count(plane_kind()); ++q) {
     void* ptr = nullptr;
     MPQC_HIP_CHECK(hipMalloc(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)));
     P.p[q] = (uint16_t*)ptr;
     plane_allocs_.push_back({P.p[q], (size_t)std::max<long>(n, 8)});
+    if (P.row) MPQC_HIP_CHECK(hipMemsetAsync(ptr, 0, (size_t)n * sizeof(uint16_t), stream_));  // the gaps stay 0
   }
   P.scale = alloc(1);
   return P;
@@ -764,6 +770,14 @@ void CCSDContext::gemmP(int M, int N, int K, double alpha, const Planes& A, long
                         long ldb, double beta, double* C, long ldc, const char* tag, int amax_slot) {
   if (M <= 0 || N <= 0 || K <= 0) throw std::logic_error("empty GEMM");
   if (lda < K || ldb < K || ldc < N) throw std::logic_error("GEMM leading dimension too small");
+  const double flops = 2.0 * M * (double)N * K;
+  if (A.row || B.row) {  // K and the leading dimensions in padded rows
+    if (A.row != B.row || K % A.row || lda % A.row || ldb % A.row)
+      throw std::logic_error(std::string("plane rows differ in ") + tag);
+    K = (int)A.at(K);
+    lda = A.at(lda);
+    ldb = B.at(ldb);
+  }
   if ((long)(M - 1) * lda + K - 1 >= A.n || (long)(N - 1) * ldb + K - 1 >= B.n)
     throw std::logic_error(std::string("out-of-bounds plane operand in ") + tag);
   check_access(C, (long)(M - 1) * ldc + (N - 1), "gemmP C");
@@ -779,7 +793,7 @@ void CCSDContext::gemmP(int M, int N, int K, double alpha, const Planes& A, long
     d.cmax_partials = partials_;
   }
   bool done = false;
-  timed(tag, 2.0 * M * (double)N * K, [&] { done = gemm_planes(d, pws_, pws_bytes_, stream_); });
+  timed(tag, flops, [&] { done = gemm_planes(d, pws_, pws_bytes_, stream_); });
   if (rec) amax_.valid[amax_slot] = done;
 }
 
@@ -787,26 +801,34 @@ void CCSDContext::gemmP(int M, int N, int K, double alpha, const Planes& A, long
 void CCSDContext::prepare_planes() {
   const long O = o_, V = v_;
   const long oovv = O * O * V * V, ovvv = O * V * V * V, vvvv = V * V * V * V, oooo = O * O * O * O;
-  // o^2 v^2 and smaller planes: every split form uses them
-  for (Planes* P : {&Gijab_P_, &GAt_P_, &GBt_P_, &GCt_P_, &tau_P_, &tauT_P_, &TP_P_, &t2P_P_, &Xjk_P_, &K_P_,
-                    &Y1t_P_, &Y2t_P_, &GbarT_P_, &Gbar_P_, &tau_ikcd_P_, &tau_ackl_P_})
-    ensure_planes(*P, oovv);
-  ensure_planes(WT_P_, oooo);
-  ensure_planes(P8T_P_, O * O * O * V);
-  ensure_planes(P13_P_, O * O * O * V);
-  ensure_planes(t1T_P_, O * V);
-  ensure_planes(gac_P_, V * V);
+  // o^2 v^2 and smaller planes: every split form uses them.  The padded row of each is the
+  // innermost index group that every contraction over it has in common.
+  const long oo = O * O, vv = V * V, ov = O * V;
+  for (Planes* P : {&Gijab_P_, &tauT_P_, &Gbar_P_, &tau_ikcd_P_}) ensure_planes(*P, oovv, vv);
+  for (Planes* P : {&tau_P_, &GbarT_P_, &tau_ackl_P_}) ensure_planes(*P, oovv, oo);
+  for (Planes* P : {&GAt_P_, &GBt_P_, &GCt_P_, &TP_P_, &t2P_P_, &Xjk_P_, &Y1t_P_}) ensure_planes(*P, oovv, ov);
+  for (Planes* P : {&K_P_, &Y2t_P_}) ensure_planes(*P, oovv, V);  // (Y2^T also as rows of c)
+  ensure_planes(WT_P_, oooo, oo);
+  ensure_planes(P8T_P_, O * O * O * V, oo);
+  ensure_planes(P13_P_, O * O * O * V, V);
+  ensure_planes(t1T_P_, O * V, V);
+  ensure_planes(gac_P_, V * V, V);
   // o v^3 planes: only where Giabc is an input (the df method builds those terms from the factors)
-  if (!df_)
-    for (Planes* P : {&Giabc_P_, &GiabcT_P_, &Gbar_akcd_P_, &P14_P_}) ensure_planes(*P, ovvv);
+  if (!df_) {
+    for (Planes* P : {&Giabc_P_, &Gbar_akcd_P_}) ensure_planes(*P, ovvv, vv);
+    for (Planes* P : {&GiabcT_P_, &P14_P_}) ensure_planes(*P, ovvv, V);
+  }
   {  // split-K workspace for the largest plane contraction shapes
     const int o = o_, v = v_;
     size_t need = 0;
-    const int shapes[][3] = {{v * v, o * o, v * v}, {o * v, o * o, v * v}, {o * o, o * o, v * v},
-                             {v * v, o * o, o * o}, {o * v, o * v, o * v}, {v, v, o * o * v},
-                             {o, o, o * v * v},     {v, o, o * v * v},     {v, o, v * o * o},
-                             {o * v * v, o, v},     {v, v * o * o, v},     {v * v, 1, o * v},
-                             {o * o, 1, o * v}};
+    // (K in padded rows)
+    const int kv = (int)plane_pitch(v), koo = (int)plane_pitch(oo), kvv = (int)plane_pitch(vv),
+              kov = (int)plane_pitch(ov);
+    const int shapes[][3] = {{v * v, o * o, kvv}, {o * v, o * o, kvv}, {o * o, o * o, kvv},
+                             {v * v, o * o, koo}, {o * v, o * v, kov}, {o * v, o * v, o * kv}, {v, v, v * koo},
+                             {o, o, o * kvv},     {v, o, o * kvv},     {v, o, v * koo},
+                             {o * v * v, o, kv},  {v, v * o * o, kv},  {v * v, 1, o * kv},
+                             {o * o, 1, o * kv}};
     for (auto& sh : shapes) need = std::max(need, gemm_planes_workspace_bytes(sh[0], sh[1], sh[2], 1));
     // the pair-symmetric ladder: v(v+1)/2 x o^2 x (v(v+1)/2 padded to 64)
     const int nvs = v * (v + 1) / 2;
@@ -829,7 +851,7 @@ void CCSDContext::prepare_planes() {
       prepare_pp_symmetric();
     } else {
       // the full contraction's v^4 planes, only where the pair-symmetric form is not usable
-      ensure_planes(Gabcd_P_, vvvv);
+      ensure_planes(Gabcd_P_, vvvv, vv);
       split(Gabcd_P_, {V, V, V, V}, {{Gabcd_, {V, V, V, V}, I, 1.0}});
     }
     split(Giabc_P_, {O, V, V, V}, {{Giabc_, {O, V, V, V}, I, 1.0}});
@@ -1135,7 +1157,7 @@ void CCSDContext::residual_ops() {
   // also stands for Rd's term (a T1 dressing term in 16-bit planes slows the split forms'
   // convergence: (H2O)8 bf16x3 36 iterations to 1e-8 instead of 18)
   auto j_giabc_t1 = [&] {
-    if (sm && !iabc_sym)
+    if (sm && !iabc_sym && !Giabc_P_.row)  // (padded rows hold (c,d) pairs, not d alone)
       gemmP(o * v * v, o, v, 1.0, Giabc_P_, v, t1T_P_, v, 0.0, Zj_, o, "r2:j_giabc_t1");
     else
       gemm(false, false, o * v * v, o, v, 1.0, Giabc_, v, t1_, o, 0.0, Zj_, o, 0, 0, 0, 1, "r2:j_giabc_t1");

@@ -244,8 +244,8 @@ class CCSDContext {
     TapePrecision& operator=(const TapePrecision&) = delete;
   };
   PlaneKind plane_kind() const;
-  Planes alloc_planes(long n);
-  void ensure_planes(Planes& P, long n);  // allocates P (n values per plane) unless it already is
+  Planes alloc_planes(long n, long row = 0);  // (rows of `row` padded to plane_pitch(row))
+  void ensure_planes(Planes& P, long n, long row);  // allocates P (n values per plane) unless it already is
   void release_planes();
   void split(const Planes& out, std::array<long, 4> n, std::initializer_list<Src> srcs,
              const TProd* prod = nullptr, const char* tag = nullptr, int line = __builtin_LINE());

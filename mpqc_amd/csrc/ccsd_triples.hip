@@ -241,7 +241,12 @@ struct DevBuf {
 struct TPlanes {
   Planes P;
   std::vector<void*> owned;
-  TPlanes(PlaneKind kind, long n) {
+  TPlanes(PlaneKind kind, long rows, long row, hipStream_t stream) {
+    if (plane_pitch(row) != row) {
+      P.row = row;
+      P.pitch = plane_pitch(row);
+    }
+    const long n = rows * plane_pitch(row);
     P.n = n;
     for (int q = 0; q < plane_count(kind); ++q) {
       void* ptr = nullptr;
@@ -252,6 +257,10 @@ struct TPlanes {
       }
       owned.push_back(ptr);
       P.p[q] = (uint16_t*)ptr;
+      if (P.row && hipMemsetAsync(ptr, 0, (size_t)n * sizeof(uint16_t), stream) != hipSuccess) {  // the gaps stay 0
+        release();
+        throw HipError("hipMemsetAsync failed");
+      }
     }
     void* sc = nullptr;
     if (hipMalloc(&sc, sizeof(double)) != hipSuccess) {
@@ -269,9 +278,10 @@ struct TPlanes {
   ~TPlanes() { release(); }
   TPlanes(const TPlanes&) = delete;
   TPlanes& operator=(const TPlanes&) = delete;
-  // the same planes starting at element `off`
+  // the same planes starting at element `off` (a whole number of rows)
   Planes at(long off) const {
     Planes q = P;
+    off = P.at(off);
     for (int k = 0; k < 3; ++k)
       if (q.p[k]) q.p[k] += off;
     q.n = P.n - off;
@@ -377,14 +387,15 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   // k-contiguous layout (A as is; B transposed to [c][K] rows), split once here
   const bool sm = split_mode();
   const PlaneKind kind = plane_kind();
+  const long VKp = plane_pitch(VK);
   std::unique_ptr<TPlanes> Ap, BTp, BT2p, BPp;
   std::unique_ptr<DevBuf> wsP;
   size_t wsP_bytes = 0;
   if (sm) {
-    Ap.reset(new TPlanes(kind, O * V * V * VK));
-    BTp.reset(new TPlanes(kind, O * O * V * VK));
-    BT2p.reset(new TPlanes(kind, O * O * V * VK));
-    BPp.reset(new TPlanes(kind, O * O * 2 * V * VK));
+    Ap.reset(new TPlanes(kind, O * V * V, VK, stream_));
+    BTp.reset(new TPlanes(kind, O * O * V, VK, stream_));
+    BT2p.reset(new TPlanes(kind, O * O * V, VK, stream_));
+    BPp.reset(new TPlanes(kind, O * O * 2 * V, VK, stream_));
     auto split1 = [&](const Planes& out, const long out_ext[4], const double* src, const long in_ext[4],
                       const int perm[4]) {
       TTerm t;
@@ -405,8 +416,8 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
     const int p_bp[4] = {0, 1, 3, 2};
     split1(BPp->P, e_bpo, Bp.p, e_bp, p_bp);    // [j][k][(t,c)][K]
     for (long nb = 1; nb <= nbmax; ++nb) {
-      wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(nb * V * V), (int)(2 * V), (int)VK, 1));
-      wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(V * V), (int)(nb * V), (int)VK, 1));
+      wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(nb * V * V), (int)(2 * V), (int)VKp, 1));
+      wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(V * V), (int)(nb * V), (int)VKp, 1));
     }
     wsP.reset(new DevBuf((wsP_bytes + sizeof(double) - 1) / sizeof(double)));
     MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
@@ -414,8 +425,8 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   auto plane_gemm = [&](int M, int N, const Planes& A, const Planes& B, double* C, long ldc) {
     PlaneGemmDesc dg;
     dg.kind = kind;
-    dg.M = M; dg.N = N; dg.K = (int)VK; dg.alpha = 1.0; dg.beta = 0.0;
-    dg.A = A; dg.lda = VK; dg.sA = 0; dg.B = B; dg.ldb = VK; dg.sB = 0;
+    dg.M = M; dg.N = N; dg.K = (int)VKp; dg.alpha = 1.0; dg.beta = 0.0;
+    dg.A = A; dg.lda = VKp; dg.sA = 0; dg.B = B; dg.ldb = VKp; dg.sB = 0;
     dg.C = C; dg.ldc = ldc; dg.sC = 0; dg.batch = 1;
     gemm_planes(dg, wsP->p, wsP_bytes, stream_);
   };

@@ -126,12 +126,16 @@ struct SplitOut {
   uint16_t* p[3];
   const double* scale;
   int kind;
+  long pad;        // pitch - row of padded planes, or 0
+  double inv_row;  // 1 / row
 };
 
 template <int SHAPE>
 __global__ __launch_bounds__(kPThreads) void split_write_kernel(PermGeom g, SplitOut o) {
   const double sc = *o.scale;
   permute_block<SHAPE>(g, blockIdx.x, blockIdx.y, blockIdx.z, [&](long e, double v) {
+    // row of e: the quotient's error, e 2^-52, is far below the half added (e < 2^50)
+    if (o.pad) e += (long)(((double)e + 0.5) * o.inv_row) * o.pad;
     const double x = v * sc;
     if (o.kind == (int)PlaneKind::F16x2) {
       const uint16_t h = f16_bits((float)x);
@@ -1212,7 +1216,8 @@ void split_to_planes(PlaneKind kind, const Planes& out, const long n[4], const T
                      AbsMaxCache* cache) {
   if (nterms < 1 || nterms > kMaxTerms) throw std::invalid_argument("split_to_planes: bad term count");
   const long total = n[0] * n[1] * n[2] * n[3];
-  if (total > out.n) throw std::invalid_argument("split_to_planes: planes too small");
+  if (out.row && total % out.row != 0) throw std::invalid_argument("split_to_planes: part of a padded row");
+  if (out.at(total) > out.n) throw std::invalid_argument("split_to_planes: planes too small");
   if (total == 0) return;
   // scale: per distinct input, max |x| (fp16 planes only)
   ScaleArgs sa{};
@@ -1263,7 +1268,8 @@ void split_to_planes(PlaneKind kind, const Planes& out, const long n[4], const T
   }
   hipLaunchKernelGGL(scale_stage2, dim3(1), dim3(256), 0, stream, partials, sa, out.scale);
   const PermGeom g = make_perm_geom(n, terms, nterms, prod);
-  SplitOut so{{out.p[0], out.p[1], out.p[2]}, out.scale, (int)kind};
+  SplitOut so{{out.p[0], out.p[1], out.p[2]}, out.scale, (int)kind, out.row ? out.pitch - out.row : 0,
+              out.row ? 1.0 / (double)out.row : 0.0};
   if (g.tiled)
     if (perm_fast_tile(g) == 3)
       hipLaunchKernelGGL(split_write_kernel<3>, perm_grid(g), dim3(kPThreads), perm_lds_bytes(g), stream, g, so);

@@ -25,7 +25,16 @@ struct Planes {
   uint16_t* p[3] = {nullptr, nullptr, nullptr};
   double* scale = nullptr;  // device scalar (power of two; 1 for bf16)
   long n = 0;               // elements per plane
+  // Row padding: every `row` consecutive elements of the tensor are stored `pitch` apart,
+  // the gap zero (0: dense).  The contractions read operand rows in 16-byte pieces, so
+  // K and the row starts have to be multiples of 8; with odd orbital counts o^2, v^2,
+  // o v are not, and a row of a contraction is made of whole padded rows instead, whose
+  // zeros add nothing when both operands are padded alike.
+  long row = 0, pitch = 0;
+  // position of a whole number of rows in the planes
+  long at(long e) const { return row ? e / row * pitch : e; }
 };
+inline long plane_pitch(long row) { return (row + 7) / 8 * 8; }
 
 // Writes planes of  out[i0,i1,i2,i3] = sum_t alpha_t in_t[...]  (permuted linear
 // combination, as tadd) with extents n; computes the scale on the device first

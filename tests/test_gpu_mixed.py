@@ -130,3 +130,35 @@ def test_deep_pipeline_plane_kernel_residual(prec):
         assert max(errs[name]) > 1e-13
     d2 = np.abs(out["dl"][1] - out["old"][1]).max() / np.abs(r2r).max()
     assert 0.0 < d2 < 2 * RES_BOUNDS[prec]     # different kernels really ran
+
+
+@pytest.mark.parametrize("prec", ["f16x3", "bf16x3", "bf16x6"])
+@pytest.mark.parametrize("no,nv,symmetric", [(7, 37, True), (5, 53, True), (6, 44, True), (8, 33, False), (1, 9, True)])
+def test_padded_plane_rows_residual(prec, no, nv, symmetric):
+    """Orbital counts whose o^2, v^2, o v or v is no multiple of 8, so the planes' rows are
+    padded: odd ones, an even v with o v a multiple of 8, one occupied orbital, and
+    integrals without Giabc(i,c,a,b) = Giabc(i,b,a,c) (its T1 term then leaves the planes);
+    against the oracle within the form's bound."""
+    from oracle import ccsd as O
+    from mpqc_amd.ccsd import CCSD, Integrals
+    from spinorb_ccsd import mpqc_blocks, random_hamiltonian
+    f, g = random_hamiltonian(no, nv, seed=no + nv, eri_scale=0.03)
+    b = mpqc_blocks(f, g, no)
+    rng = np.random.default_rng(no * nv)
+    if not symmetric:
+        b["Giabc"] = b["Giabc"] + rng.normal(0, 0.01, b["Giabc"].shape)
+    t1 = rng.normal(0, 0.01, (nv, no))
+    t2 = rng.normal(0, 0.01, (nv, nv, no, no))
+    ints = O.Integrals(**b)
+    tau = O.make_tau(t1, t2)
+    r1r = O.cs_ccsd_r1(t1, t2, tau, ints)
+    r2r = O.cs_ccsd_r2(t1, t2, tau, ints)
+    with CCSD(no, nv, precision=prec) as c:
+        c.set_integrals(Integrals(**b))
+        c.set_orbital_energies(np.diag(f)[:no], np.diag(f)[no:])
+        c.compute_residuals(0.5 * t1, 0.5 * t2)  # the planes are written again
+        r1, r2 = c.compute_residuals(t1, t2)
+    e1 = np.abs(r1 - r1r).max() / np.abs(r1r).max()
+    e2 = np.abs(r2 - r2r).max() / np.abs(r2r).max()
+    print(f"{prec} o={no} v={nv}: rel err r1 {e1:.2e} r2 {e2:.2e}")
+    assert e1 < RES_BOUNDS[prec] and e2 < RES_BOUNDS[prec]

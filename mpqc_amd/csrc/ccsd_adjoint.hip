@@ -51,10 +51,7 @@ double* CCSDContext::adj(const double* p) {
   if (adj_.size() < allocations_.size()) adj_.resize(allocations_.size(), nullptr);
   if (!adj_[k]) {
     void* q = nullptr;
-    if (hipMalloc(&q, alloc_sizes_[k] * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      throw std::bad_alloc();
-    }
+    if (scratch_.allocate(&q, alloc_sizes_[k] * sizeof(double)) != hipSuccess) throw std::bad_alloc();
     adj_[k] = (double*)q;
     fill(adj_[k], (long)alloc_sizes_[k], 0.0, stream_);
   }
@@ -73,7 +70,7 @@ double* CCSDContext::adj_scratch(long n) {
   if (adj_scratch_n_ < n) {
     if (adj_scratch_) MPQC_HIP_CHECK(hipFree(adj_scratch_));
     adj_scratch_ = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&adj_scratch_, n * sizeof(double)));
+    MPQC_HIP_CHECK(scratch_.allocate((void**)&adj_scratch_, n * sizeof(double)));
     adj_scratch_n_ = n;
   }
   return adj_scratch_;
@@ -193,7 +190,7 @@ void CCSDContext::reverse_op(const TapeOp& op, bool integrals) {
           if (adj_ws_n_ < need) {
             if (adj_ws_) MPQC_HIP_CHECK(hipFree(adj_ws_));
             adj_ws_ = nullptr;
-            MPQC_HIP_CHECK(hipMalloc(&adj_ws_, need * sizeof(double)));
+            MPQC_HIP_CHECK(scratch_.allocate((void**)&adj_ws_, need * sizeof(double)));
             adj_ws_n_ = need;
           }
           d.C = adj_ws_;

@@ -101,6 +101,7 @@ CCSDContext::CCSDContext(int o, int v, const int64_t* occ_hm, int n_occ_tiles, c
 
 void CCSDContext::release() {
   if (stream_) hipStreamSynchronize(stream_);
+  scratch_.clear();
   drop_residual_graph();
   for (auto& pe : pending_) {
     hipEventDestroy(pe.a);
@@ -189,11 +190,7 @@ CCSDContext::~CCSDContext() { release(); }
 
 double* CCSDContext::alloc(size_t n) {
   void* p = nullptr;
-  hipError_t e = hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(double));
-  if (e != hipSuccess) {
-    (void)hipGetLastError();
-    throw std::bad_alloc();
-  }
+  if (scratch_.allocate(&p, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   allocations_.push_back((double*)p);
   alloc_sizes_.push_back(std::max<size_t>(n, 1));
   return (double*)p;
@@ -334,7 +331,7 @@ void CCSDContext::upload(double* dst, const double* src, const std::array<int, 4
     if (staging_n_ < (size_t)total) {
       if (staging_) MPQC_HIP_CHECK(hipFree(staging_));
       staging_ = nullptr;
-      MPQC_HIP_CHECK(hipMalloc(&staging_, total * sizeof(double)));
+      MPQC_HIP_CHECK(scratch_.allocate((void**)&staging_, total * sizeof(double)));
       staging_n_ = total;
     }
     MPQC_HIP_CHECK(hipMemcpyAsync(staging_, src, total * sizeof(double), hipMemcpyHostToDevice, stream_));
@@ -402,7 +399,7 @@ void CCSDContext::download(double* dst, const double* src, const std::array<int,
     if (staging_n_ < (size_t)total) {
       if (staging_) MPQC_HIP_CHECK(hipFree(staging_));
       staging_ = nullptr;
-      MPQC_HIP_CHECK(hipMalloc(&staging_, total * sizeof(double)));
+      MPQC_HIP_CHECK(scratch_.allocate((void**)&staging_, total * sizeof(double)));
       staging_n_ = total;
     }
     ddst = staging_;
@@ -746,7 +743,7 @@ Planes CCSDContext::alloc_planes(long n, long row) {
   P.n = n;
   for (int q = 0; q < plane_count(plane_kind()); ++q) {
     void* ptr = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)));
+    MPQC_HIP_CHECK(scratch_.allocate(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)));
     P.p[q] = (uint16_t*)ptr;
     plane_allocs_.push_back({P.p[q], (size_t)std::max<long>(n, 8)});
     if (P.row) MPQC_HIP_CHECK(hipMemsetAsync(ptr, 0, (size_t)n * sizeof(uint16_t), stream_));  // the gaps stay 0

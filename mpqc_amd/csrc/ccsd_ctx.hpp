@@ -10,6 +10,7 @@
 #include "common.hpp"
 #include "gemm.hpp"
 #include "planes.hpp"
+#include "scratch.hpp"
 #include "tensor_ops.hpp"
 
 namespace mpqc_hip {
@@ -289,6 +290,7 @@ class CCSDContext {
   std::vector<int64_t> occ_hm_, vir_hm_;
   std::vector<double*> allocations_;
   std::vector<size_t> alloc_sizes_;
+  ScratchCache scratch_;  // temporaries of transform_ao / transform_df and triples
 
   // density fitting (method "df"): three-index factors X(K,p,q) and their layouts
   bool df_ = false, reduced_abcd_ = true;

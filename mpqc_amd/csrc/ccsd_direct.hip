@@ -20,6 +20,7 @@ void CCSDContext::set_direct_ao(int nbf, const double* ao_eri, const double* c_o
                                 int memspace) {
   if (nbf <= 0 || !ao_eri || !c_occ || !c_vir) throw std::invalid_argument("set_direct_ao: null or empty input");
   if (memspace != 0 && memspace != 1) throw std::invalid_argument("memspace must be host or device");
+  if (memspace) MPQC_HIP_CHECK(hipDeviceSynchronize());  // the caller's pending work on its buffers
   const long n = nbf, O = o_, V = v_, oo = O * O;
   if (O + V > n) throw std::invalid_argument("more active orbitals than basis functions");
   if (n * n * n * n >= (1L << 31)) throw std::invalid_argument("nbf^4 must be < 2^31 for the direct method");
@@ -43,10 +44,7 @@ void CCSDContext::set_direct_ao(int nbf, const double* ao_eri, const double* c_o
   const long n4 = n * n * n * n;
   double* src = nullptr;
   if (!memspace) {
-    if (hipMalloc(&src, (size_t)n4 * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      throw std::bad_alloc();
-    }
+    if (scratch_.allocate((void**)&src, (size_t)n4 * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   }
   try {
     if (!memspace)

@@ -132,10 +132,7 @@ void CCSDContext::ensure_abcd_from_factors() {
   const long Q = naux_, V = v_, vv = V * V;
   if (!Gabcd_) Gabcd_ = alloc((size_t)vv * vv);
   double* T = nullptr;
-  if (hipMalloc(&T, (size_t)vv * vv * sizeof(double)) != hipSuccess) {
-    (void)hipGetLastError();
-    throw std::bad_alloc();
-  }
+  if (scratch_.allocate((void**)&T, (size_t)vv * vv * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   try {
     mpqc_hip::gemm(make_gemm(true, false, (int)vv, (int)vv, (int)Q, 1.0, Xab_, vv, Xab_, vv, 0.0, T, vv),
                    GemmPrecision::F64, ws_, stream_);
@@ -176,6 +173,7 @@ void CCSDContext::eom_apply_jt(const double* y, double* x) {
 }
 
 int CCSDContext::eom_ee(int n_roots, int max_iter, double convergence, int verbose, double* energies) {
+  scratch_.clear();  // (the vector pool may need the memory)
   if (n_roots < 1) throw std::invalid_argument("n_roots must be positive");
   if (max_iter < 1) throw std::invalid_argument("max_iter must be positive");
   if (!(convergence > 0.0)) throw std::invalid_argument("convergence must be positive");

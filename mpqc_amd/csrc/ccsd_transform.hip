@@ -10,7 +10,7 @@
 // are <p|F|q> = C_p^T F C_q.
 //
 // Both entry points write the context's integral buffers exactly as
-// set_integral would; temporaries are allocated for the call and released.
+// set_integral would; temporaries come from the context's scratch cache.
 #include <stdexcept>
 
 #include "ccsd_ctx.hpp"
@@ -18,23 +18,6 @@
 namespace mpqc_hip {
 
 namespace {
-
-struct DevTmp {
-  double* p = nullptr;
-  explicit DevTmp(size_t n) {
-    if (n == 0) return;
-    if (hipMalloc(&p, n * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
-      throw std::bad_alloc();
-    }
-  }
-  ~DevTmp() {
-    if (p) (void)hipFree(p);
-  }
-  DevTmp(const DevTmp&) = delete;
-  DevTmp& operator=(const DevTmp&) = delete;
-};
 
 // out[a,b,c,d] (extents n) = src[off + a*s0 + b*s1 + c*s2 + d*s3]
 void strided_copy(double* out, const long n[4], const double* src, long off, const long s[4], long src_vol,
@@ -67,7 +50,7 @@ static void gather_coefficients(double* Cact, int nbf, int o, int v, const doubl
 // Fia, Fij, Fab = blocks of C_act^T F C_act  (<i|F|a>, <i|F|j>, <a|F|b>)
 void CCSDContext::transform_fock(int nbf, const double* fock, const double* Cact, int memspace) {
   const int o = o_, v = v_, nmo = o_ + v_;
-  DevTmp Fdev(memspace ? 0 : (size_t)nbf * nbf), T((size_t)nbf * nmo), Fmo((size_t)nmo * nmo);
+  ScratchBuf Fdev(scratch_, memspace ? 0 : (size_t)nbf * nbf), T(scratch_, (size_t)nbf * nmo), Fmo(scratch_, (size_t)nmo * nmo);
   const double* F = fock;
   if (!memspace) {
     MPQC_HIP_CHECK(hipMemcpyAsync(Fdev.p, fock, (size_t)nbf * nbf * sizeof(double), hipMemcpyHostToDevice, stream_));
@@ -95,23 +78,24 @@ void CCSDContext::transform_ao(int nbf, const double* eri, const double* fock, c
                                const double* c_vir, int memspace) {
   if (nbf <= 0 || !eri || !fock || !c_occ || !c_vir) throw std::invalid_argument("transform_ao: null or empty input");
   if (memspace != 0 && memspace != 1) throw std::invalid_argument("memspace must be host or device");
+  if (memspace) MPQC_HIP_CHECK(hipDeviceSynchronize());  // the caller's pending work on its buffers
   const long n = nbf, nmo = (long)o_ + v_, O = o_, V = v_;
   if (nmo > n) throw std::invalid_argument("more active orbitals than basis functions");
   if (n * n * n >= (1L << 31) || n * n * n * n >= (1L << 40))
     throw std::invalid_argument("nbf too large for the dense AO transform");
   const long n4 = n * n * n * n;
-  DevTmp Cact((size_t)n * nmo);
+  ScratchBuf Cact(scratch_, (size_t)n * nmo);
   gather_coefficients(Cact.p, nbf, o_, v_, c_occ, c_vir, memspace, stream_);
   // buffers: x0 = AO (caller's device buffer or an upload), bufA for (nu la si p) and
   // (si p q r), bufB for (la si p q) and (p q r s)
-  DevTmp up(memspace ? 0 : (size_t)n4);
+  ScratchBuf up(scratch_, memspace ? 0 : (size_t)n4);
   const double* x0 = eri;
   if (!memspace) {
     MPQC_HIP_CHECK(hipMemcpyAsync(up.p, eri, n4 * sizeof(double), hipMemcpyHostToDevice, stream_));
     x0 = up.p;
   }
-  DevTmp bufA((size_t)std::max(n * n * n * nmo, n * nmo * nmo * nmo));
-  DevTmp bufB(memspace ? (size_t)std::max(n * n * nmo * nmo, nmo * nmo * nmo * nmo) : 0);
+  ScratchBuf bufA(scratch_, (size_t)std::max(n * n * n * nmo, n * nmo * nmo * nmo));
+  ScratchBuf bufB(scratch_, memspace ? (size_t)std::max(n * n * nmo * nmo, nmo * nmo * nmo * nmo) : 0);
   double* pB = memspace ? bufB.p : up.p;  // the uploaded AO buffer is free after the first quarter
   auto quarter = [&](const double* x, double* y, long rest) {
     // y[(rest), p] = sum_mu x[mu, (rest)] C[mu, p]
@@ -152,14 +136,16 @@ void CCSDContext::transform_df(int nbf, const double* B3, const double* metric, 
   if (naux_ == 0) throw std::logic_error("transform_df needs set_df_basis first");
   if (nbf <= 0 || !B3 || !fock || !c_occ || !c_vir) throw std::invalid_argument("transform_df: null or empty input");
   if (memspace != 0 && memspace != 1) throw std::invalid_argument("memspace must be host or device");
+  if (memspace) MPQC_HIP_CHECK(hipDeviceSynchronize());  // the caller's pending work on its buffers
   const long n = nbf, Q = naux_, nmo = (long)o_ + v_, O = o_, V = v_;
   if (nmo > n) throw std::invalid_argument("more active orbitals than basis functions");
   if (Q * n * n >= (1L << 31)) throw std::invalid_argument("naux * nbf^2 too large");
   const hipMemcpyKind kind = memspace ? hipMemcpyDeviceToDevice : hipMemcpyHostToDevice;
-  DevTmp Cact((size_t)n * nmo);
+  ScratchBuf Cact(scratch_, (size_t)n * nmo);
   gather_coefficients(Cact.p, nbf, o_, v_, c_occ, c_vir, memspace, stream_);
   // fitted AO factors X(K, mu nu) = sum_L metric(L,K) B(L, mu nu)
-  DevTmp Xao((size_t)Q * n * n), Bup(metric ? (size_t)Q * n * n : 0), Mup(metric ? (size_t)Q * Q : 0);
+  ScratchBuf Xao(scratch_, (size_t)Q * n * n), Bup(scratch_, metric ? (size_t)Q * n * n : 0),
+      Mup(scratch_, metric ? (size_t)Q * Q : 0);
   if (metric) {
     MPQC_HIP_CHECK(hipMemcpyAsync(Bup.p, B3, Q * n * n * sizeof(double), kind, stream_));
     MPQC_HIP_CHECK(hipMemcpyAsync(Mup.p, metric, Q * Q * sizeof(double), kind, stream_));
@@ -169,7 +155,7 @@ void CCSDContext::transform_df(int nbf, const double* B3, const double* metric, 
     MPQC_HIP_CHECK(hipMemcpyAsync(Xao.p, B3, Q * n * n * sizeof(double), kind, stream_));
   }
   // Y(K,mu,q) = X(K,mu,nu) C(nu,q);  Z(K,p,q) = C(mu,p) Y(K,mu,q)
-  DevTmp Y((size_t)Q * n * nmo), Z((size_t)Q * nmo * nmo);
+  ScratchBuf Y(scratch_, (size_t)Q * n * nmo), Z(scratch_, (size_t)Q * nmo * nmo);
   mpqc_hip::gemm(make_gemm(false, false, (int)(Q * n), (int)nmo, nbf, 1.0, Xao.p, n, Cact.p, nmo, 0.0, Y.p, nmo),
                  GemmPrecision::F64, ws_, stream_);
   {
@@ -187,14 +173,14 @@ void CCSDContext::transform_df(int nbf, const double* B3, const double* metric, 
   }
   // Xia(K,i,a) contiguous, then the four-index blocks as X^T X GEMMs over K and one
   // permutation each
-  DevTmp Xia((size_t)Q * O * V);
+  ScratchBuf Xia(scratch_, (size_t)Q * O * V);
   {
     const long e_ia[4] = {1, Q, O, V};
     strided_copy(Xia.p, e_ia, Z.p, O, zs, zvol, stream_);
   }
   const bool full = !reduced_abcd_;
   const long tmp_n = full ? std::max(V * V * V * V, O * V * V * V) : std::max(O * O * V * V, O * O * O * V);
-  DevTmp T((size_t)std::max(tmp_n, O * O * O * O));
+  ScratchBuf T(scratch_, (size_t)std::max(tmp_n, O * O * O * O));
   // dst[perm(x,y,z,w)] = sum_K A(K,x,y) B(K,z,w): T[(x,y)][(z,w)] = A^T B, then dst = permute(T)
   auto block = [&](double* dst, const double* A, long nx, long ny, const double* Bm, long nz, long nw,
                    std::array<int, 4> perm) {

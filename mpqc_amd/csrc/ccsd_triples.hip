@@ -221,27 +221,11 @@ __global__ __launch_bounds__(256) void sum_to_slot(const double* partials, long 
   if (threadIdx.x == 0) acc[slot] = sh[0];
 }
 
-struct DevBuf {
-  double* p = nullptr;
-  explicit DevBuf(size_t n) {
-    if (hipMalloc(&p, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      p = nullptr;
-      throw std::bad_alloc();
-    }
-  }
-  ~DevBuf() {
-    if (p) (void)hipFree(p);
-  }
-  DevBuf(const DevBuf&) = delete;
-  DevBuf& operator=(const DevBuf&) = delete;
-};
-
 // planes of one (T) operand, owned for the duration of the call
 struct TPlanes {
   Planes P;
-  std::vector<void*> owned;
-  TPlanes(PlaneKind kind, long rows, long row, hipStream_t stream) {
+  std::vector<std::unique_ptr<ScratchBuf>> owned;
+  TPlanes(ScratchCache& scratch, PlaneKind kind, long rows, long row, hipStream_t stream) {
     if (plane_pitch(row) != row) {
       P.row = row;
       P.pitch = plane_pitch(row);
@@ -249,35 +233,13 @@ struct TPlanes {
     const long n = rows * plane_pitch(row);
     P.n = n;
     for (int q = 0; q < plane_count(kind); ++q) {
-      void* ptr = nullptr;
-      if (hipMalloc(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)) != hipSuccess) {
-        (void)hipGetLastError();
-        release();
-        throw std::bad_alloc();
-      }
-      owned.push_back(ptr);
-      P.p[q] = (uint16_t*)ptr;
-      if (P.row && hipMemsetAsync(ptr, 0, (size_t)n * sizeof(uint16_t), stream) != hipSuccess) {  // the gaps stay 0
-        release();
-        throw HipError("hipMemsetAsync failed");
-      }
+      owned.emplace_back(new ScratchBuf(scratch, (size_t)ceil_div(std::max<long>(n, 8), 4)));
+      P.p[q] = (uint16_t*)owned.back()->p;
+      if (P.row) MPQC_HIP_CHECK(hipMemsetAsync(P.p[q], 0, (size_t)n * sizeof(uint16_t), stream));  // the gaps stay 0
     }
-    void* sc = nullptr;
-    if (hipMalloc(&sc, sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      release();
-      throw std::bad_alloc();
-    }
-    owned.push_back(sc);
-    P.scale = (double*)sc;
+    owned.emplace_back(new ScratchBuf(scratch, 1));
+    P.scale = owned.back()->p;
   }
-  void release() {
-    for (void* x : owned) (void)hipFree(x);
-    owned.clear();
-  }
-  ~TPlanes() { release(); }
-  TPlanes(const TPlanes&) = delete;
-  TPlanes& operator=(const TPlanes&) = delete;
   // the same planes starting at element `off` (a whole number of rows)
   Planes at(long off) const {
     Planes q = P;
@@ -309,7 +271,7 @@ void CCSDContext::ensure_iabc_for_triples() {
   if ((have_ints_ >> 6) & 1u) return;
   if (!df_) throw std::logic_error("(T) needs Giabc");
   const long Q = naux_, O = o_, V = v_;
-  DevBuf T((size_t)(O * V * V * V));
+  ScratchBuf T(scratch_, (size_t)(O * V * V * V));
   // T[(i,b)][(a,c)] = Xia(K,(i,b))^T Xab(K,(a,c)) ; Giabc(i,a,b,c) = T(i,b,a,c)
   mpqc_hip::gemm(make_gemm(true, false, (int)(O * V), (int)(V * V), (int)Q, 1.0, Xia_, O * V, Xab_, V * V, 0.0,
                            T.p, V * V), GemmPrecision::F64, ws_, stream_);
@@ -342,10 +304,11 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   // and three layouts of Bcat that make the N dimension of each GEMM long:
   //   Bt (K, j, k, c), Bt2 (K, k, j, c) = Bcat(j, k, K, c), Bp (j, k, K, 2, c) = [Bcat(j,k) | Bcat(k,j)]
   const size_t d = sizeof(double);
-  DevBuf Acat((size_t)(O * V * V * VK)), Bt((size_t)(VK * O * O * V)), Bt2((size_t)(VK * O * O * V)),
-      Bp((size_t)(2 * O * O * VK * V)), W((size_t)(6 * nbmax * v3));
+  ScratchBuf Acat(scratch_, (size_t)(O * V * V * VK)), Bt(scratch_, (size_t)(VK * O * O * V)),
+      Bt2(scratch_, (size_t)(VK * O * O * V)), Bp(scratch_, (size_t)(2 * O * O * VK * V)),
+      W(scratch_, (size_t)(6 * nbmax * v3));
   {
-    DevBuf tmp((size_t)(O * V * V * std::max(V, O)));
+    ScratchBuf tmp(scratch_, (size_t)(O * V * V * std::max(V, O)));
     // Acat[i][(a,b)][d] = Giabc(i,d,a,b); Acat[i][(a,b)][v + l] = t2(a,b,i,l)
     const long e_iabc[4] = {O, V, V, V};
     const int p1[4] = {0, 2, 3, 1};
@@ -359,7 +322,7 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
     MPQC_HIP_CHECK(hipMemcpy2DAsync(Acat.p + V, VK * d, tmp.p, O * d, O * d, O * V * V, hipMemcpyDeviceToDevice,
                                     stream_));
     // Bcat[j][k][d][c] = t2(d,c,j,k); Bcat[j][k][v + l][c] = -Gijka(j,k,l,c)
-    DevBuf Bcat((size_t)(O * O * VK * V)), tmp2((size_t)(O * O * std::max(V, O) * V));
+    ScratchBuf Bcat(scratch_, (size_t)(O * O * VK * V)), tmp2(scratch_, (size_t)(O * O * std::max(V, O) * V));
     const int p3[4] = {2, 3, 0, 1};
     const long ext3[4] = {O, O, V, V};
     permute_into(tmp2.p, ext3, t2_, e_t2, p3, 1.0, stream_);
@@ -377,11 +340,10 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
     permute_into(Bt2.p, e_bt, Bcat.p, e_b, pt2, 1.0, stream_);
     MPQC_HIP_CHECK(hipMemcpy2DAsync(Bp.p, 2 * V * d, Bcat.p, V * d, V * d, O * O * VK, hipMemcpyDeviceToDevice,
                                     stream_));
-    DevBuf BcatT((size_t)(O * O * VK * V));
+    ScratchBuf BcatT(scratch_, (size_t)(O * O * VK * V));
     permute_into(BcatT.p, e_b, Bcat.p, e_b, psw, 1.0, stream_);  // BcatT(j,k) = Bcat(k,j)
     MPQC_HIP_CHECK(hipMemcpy2DAsync(Bp.p + V, 2 * V * d, BcatT.p, V * d, V * d, O * O * VK,
                                     hipMemcpyDeviceToDevice, stream_));
-    MPQC_HIP_CHECK(hipStreamSynchronize(stream_));  // temporaries are released on return
   }
   // split-precision forms: the W GEMMs read 16-bit planes of the operands in
   // k-contiguous layout (A as is; B transposed to [c][K] rows), split once here
@@ -389,13 +351,13 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   const PlaneKind kind = plane_kind();
   const long VKp = plane_pitch(VK);
   std::unique_ptr<TPlanes> Ap, BTp, BT2p, BPp;
-  std::unique_ptr<DevBuf> wsP;
+  std::unique_ptr<ScratchBuf> wsP;
   size_t wsP_bytes = 0;
   if (sm) {
-    Ap.reset(new TPlanes(kind, O * V * V, VK, stream_));
-    BTp.reset(new TPlanes(kind, O * O * V, VK, stream_));
-    BT2p.reset(new TPlanes(kind, O * O * V, VK, stream_));
-    BPp.reset(new TPlanes(kind, O * O * 2 * V, VK, stream_));
+    Ap.reset(new TPlanes(scratch_, kind, O * V * V, VK, stream_));
+    BTp.reset(new TPlanes(scratch_, kind, O * O * V, VK, stream_));
+    BT2p.reset(new TPlanes(scratch_, kind, O * O * V, VK, stream_));
+    BPp.reset(new TPlanes(scratch_, kind, O * O * 2 * V, VK, stream_));
     auto split1 = [&](const Planes& out, const long out_ext[4], const double* src, const long in_ext[4],
                       const int perm[4]) {
       TTerm t;
@@ -419,7 +381,7 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
       wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(nb * V * V), (int)(2 * V), (int)VKp, 1));
       wsP_bytes = std::max(wsP_bytes, gemm_planes_workspace_bytes((int)(V * V), (int)(nb * V), (int)VKp, 1));
     }
-    wsP.reset(new DevBuf((wsP_bytes + sizeof(double) - 1) / sizeof(double)));
+    wsP.reset(new ScratchBuf(scratch_, (wsP_bytes + sizeof(double) - 1) / sizeof(double)));
     MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
   }
   auto plane_gemm = [&](int M, int N, const Planes& A, const Planes& B, double* C, long ldc) {
@@ -439,7 +401,7 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   long nchunks = 0;
   for (int k = 0; k < o; ++k)
     for (int j = 0; j <= k; ++j) nchunks += ceil_div(j + 1, nbmax);
-  DevBuf partials((size_t)(ncube * nbmax)), acc((size_t)nchunks);
+  ScratchBuf partials(scratch_, (size_t)(ncube * nbmax)), acc(scratch_, (size_t)nchunks);
   long slot = 0;
   for (int k = 0; k < o; ++k)
     for (int j = 0; j <= k; ++j)

@@ -69,11 +69,18 @@ void CCSDContext::transform_fock(int nbf, const double* fock, const double* Cact
   have_ints_ |= 0x7u;
 }
 
-// compute4 without density fitting (lcao_factory.h:421-493): four quarter
-// transforms of (mu nu|la si) by C_act, each one GEMM that contracts the
-// leading index and appends the new one, (mu nu la si) -> (nu la si p) -> ...
-// -> (p q r s); then the physical blocks <PQ|RS>[a,b,c,d] = (p=P0+a, q=R0+c |
-// r=Q0+b, s=S0+d) by strided copies.
+// compute4 without density fitting (lcao_factory.h:421-493): quarter transforms of
+// (mu nu|la si), each one GEMM that contracts an index and appends the new one, in the
+// order mu -> p, la -> r, nu -> q, si -> s.  In that order a block <pr|qs> = (pq|rs) with
+// p, r, q, s occupied or virtual comes out of the last GEMM in its own layout:
+//   (mu nu la si) -> Y1 (nu la si p) -> Y2 (nu si p r) -> Y3 (si p r q) -> <pr|qs>,
+// and the tree of occupied / virtual choices stops at the six blocks that are needed:
+// p = i: r = j: q = k: <ij|kl>, <ij|ka>; q = a: <ij|ab>; r = a: q = j: <ia|jb>; q = b: <ia|bc>;
+// p = a: r = b: q = c: <ab|cd>.  (All of (pq|rs) and six strided copies took 2.5e11 multiply-adds
+// and 9 GB at 144 functions and 30 + 114 orbitals; the tree takes 1.95e11 and 5 GB.)  p goes in
+// blocks and nu in slabs, so that Y1 to Y3 fit the scratch cache and calls after the first
+// allocate nothing.  Bound: the matrix cores (at
+// those sizes 15.0 -> 9.8 ms of kernels, 40 TFLOP/s, and 101-219 -> 10.6 ms for the call).
 void CCSDContext::transform_ao(int nbf, const double* eri, const double* fock, const double* c_occ,
                                const double* c_vir, int memspace) {
   if (nbf <= 0 || !eri || !fock || !c_occ || !c_vir) throw std::invalid_argument("transform_ao: null or empty input");
@@ -86,39 +93,68 @@ void CCSDContext::transform_ao(int nbf, const double* eri, const double* fock, c
   const long n4 = n * n * n * n;
   ScratchBuf Cact(scratch_, (size_t)n * nmo);
   gather_coefficients(Cact.p, nbf, o_, v_, c_occ, c_vir, memspace, stream_);
-  // buffers: x0 = AO (caller's device buffer or an upload), bufA for (nu la si p) and
-  // (si p q r), bufB for (la si p q) and (p q r s)
   ScratchBuf up(scratch_, memspace ? 0 : (size_t)n4);
   const double* x0 = eri;
   if (!memspace) {
     MPQC_HIP_CHECK(hipMemcpyAsync(up.p, eri, n4 * sizeof(double), hipMemcpyHostToDevice, stream_));
     x0 = up.p;
   }
-  ScratchBuf bufA(scratch_, (size_t)std::max(n * n * n * nmo, n * nmo * nmo * nmo));
-  ScratchBuf bufB(scratch_, memspace ? (size_t)std::max(n * n * nmo * nmo, nmo * nmo * nmo * nmo) : 0);
-  double* pB = memspace ? bufB.p : up.p;  // the uploaded AO buffer is free after the first quarter
-  auto quarter = [&](const double* x, double* y, long rest) {
-    // y[(rest), p] = sum_mu x[mu, (rest)] C[mu, p]
-    mpqc_hip::gemm(make_gemm(true, false, (int)rest, (int)nmo, nbf, 1.0, x, rest, Cact.p, nmo, 0.0, y, nmo),
-                   GemmPrecision::F64, ws_, stream_);
-  };
-  quarter(x0, bufA.p, n * n * n);              // (nu la si p)
-  quarter(bufA.p, pB, n * n * nmo);            // (la si p q)
-  quarter(pB, bufA.p, n * nmo * nmo);          // (si p q r)
-  quarter(bufA.p, pB, nmo * nmo * nmo);        // (p q r s)
-  const double* mo = pB;
-  const long mo_vol = nmo * nmo * nmo * nmo;
   if (!Gabcd_) Gabcd_ = alloc((size_t)V * V * V * V);
-  struct Blk { double* dst; long P0, Q0, R0, S0, nP, nQ, nR, nS; };
-  const Blk blocks[] = {{Gijab_, 0, 0, O, O, O, O, V, V}, {Gijkl_, 0, 0, 0, 0, O, O, O, O},
-                        {Giajb_, 0, O, 0, O, O, V, O, V}, {Giabc_, 0, O, O, O, O, V, V, V},
-                        {Gijka_, 0, 0, 0, O, O, O, O, V}, {Gabcd_, O, O, O, O, V, V, V, V}};
-  for (const Blk& b : blocks) {
-    // <PQ|RS>[a,b,c,d] = mo[P0+a, R0+c, Q0+b, S0+d]
-    const long ext[4] = {b.nP, b.nQ, b.nR, b.nS};
-    const long s[4] = {nmo * nmo * nmo, nmo, nmo * nmo, 1};
-    const long off = b.P0 * nmo * nmo * nmo + b.R0 * nmo * nmo + b.Q0 * nmo + b.S0;
-    strided_copy(b.dst, ext, mo, off, s, mo_vol, stream_);
+  // out[m, c] = sum_k x[k, m] Cact[k, c0 + c], c < nc, for each of `batch` x and out
+  auto quarter = [&](const double* x, long rows, long ldx, long c0, long nc, double* out, long batch, long sx, long so) {
+    GemmDesc g = make_gemm(true, false, (int)rows, (int)nc, nbf, 1.0, x, ldx, Cact.p + c0, nmo, 0.0, out, nc);
+    g.sA = sx; g.sC = so; g.batch = (int)batch;
+    mpqc_hip::gemm(g, GemmPrecision::F64, ws_, stream_);
+  };
+  // Y1 to Y3 take 2 GiB (every p block reads the AO integrals again, but a new context's first
+  // call pays 20 to 90 ms per GB for the allocation), 128 MiB of them for Y1
+  const long kSlab = 16L << 20, budget = (256L << 20) - kSlab;
+  struct Part { long nP, nR, nRQ, pb, slab; };  // p occupied, p virtual
+  Part part[2];
+  size_t words = 0;
+  for (int virt = 0; virt < 2; ++virt) {
+    Part& t = part[virt];
+    t.nP = virt ? V : O;
+    t.nR = virt ? V : nmo;  // r: all of Y2's last index (occupied first); only virtual ones for <ab|cd>
+    t.nRQ = virt ? V * V : std::max(O, V) * std::max(O, V);
+    const long per_p = n * n * t.nR + n * t.nRQ;
+    t.pb = ceil_div(t.nP, ceil_div(t.nP, std::max(1L, budget / per_p)));
+    t.slab = std::max(1L, std::min(n, kSlab / (n * n * t.pb)));
+    words = std::max<size_t>(words, (size_t)(t.slab * n * n * t.pb + t.pb * per_p));
+  }
+  ScratchBuf Y(scratch_, words);
+  for (int virt = 0; virt < 2; ++virt) {
+    const Part& t = part[virt];
+    const long nP = t.nP, c0 = virt ? O : 0, pb = t.pb, slab = t.slab;
+    double* const Y1 = Y.p;
+    double* const Y2 = Y1 + slab * n * n * pb;
+    double* const Y3 = Y2 + n * n * pb * t.nR;
+    for (long p0 = 0; p0 < nP; p0 += pb) {
+      const long np = std::min(pb, nP - p0);
+      double* Y2o = Y2;                                  // r occupied (p occupied only)
+      double* Y2v = Y2 + (virt ? 0 : n * n * np * O);    // r virtual
+      for (long m0 = 0; m0 < n; m0 += slab) {
+        const long ns = std::min(slab, n - m0);
+        quarter(x0 + m0 * n * n, ns * n * n, n * n * n, c0 + p0, np, Y1, 1, 0, 0);
+        if (!virt) quarter(Y1, n * np, n * np, 0, O, Y2o + m0 * n * np * O, ns, n * n * np, n * np * O);
+        quarter(Y1, n * np, n * np, O, V, Y2v + m0 * n * np * V, ns, n * n * np, n * np * V);
+      }
+      // the last two quarters of one choice of r and q, to the block(s) <pr|q.>
+      auto finish = [&](const double* y2, long R, long q0, long Q, double* dst_o, double* dst_v) {
+        quarter(y2, n * np * R, n * np * R, q0, Q, Y3, 1, 0, 0);
+        const long rows = np * R * Q;
+        if (dst_o) quarter(Y3, rows, rows, 0, O, dst_o + p0 * R * Q * O, 1, 0, 0);
+        quarter(Y3, rows, rows, O, V, dst_v + p0 * R * Q * V, 1, 0, 0);
+      };
+      if (virt) {
+        finish(Y2v, V, O, V, nullptr, Gabcd_);
+      } else {
+        finish(Y2o, O, 0, O, Gijkl_, Gijka_);
+        finish(Y2o, O, O, V, nullptr, Gijab_);
+        finish(Y2v, V, 0, O, nullptr, Giajb_);
+        finish(Y2v, V, O, V, nullptr, Giabc_);
+      }
+    }
   }
   check_launch("transform_ao");
   MPQC_HIP_CHECK(hipStreamSynchronize(stream_));

@@ -126,3 +126,34 @@ def test_transform_df_matches_oracle_and_golden(reduced):
         c.set_df_basis(naux)
         c.transform_df(Xf, None, s.F, Ci, Ca)
         assert _rel(c.get_integral("Gijab"), ref["Gijab"]) < 1e-12
+
+
+@pytest.mark.parametrize("nbf,o,v", [(15, 9, 4), (96, 11, 80), (120, 8, 100)])
+def test_transform_ao_blocks_and_slabs(nbf, o, v):
+    """More occupied than virtual orbitals; several slabs of the first AO index; several blocks of
+    the first orbital.  AO "integrals" without any permutational symmetry, device buffers,
+    against torch in float64 (the file's bar)."""
+    import ctypes
+    import torch
+    from mpqc_amd import _lib as L
+    from mpqc_amd.ccsd import CCSD
+    gen = torch.Generator(device="cuda").manual_seed(nbf)
+    new = lambda *s: torch.randn(s, dtype=torch.float64, device="cuda", generator=gen)
+    eri, F, Ci, Ca = new(nbf, nbf, nbf, nbf), new(nbf, nbf), new(nbf, o), new(nbf, v)
+    C = torch.cat([Ci, Ca], 1)
+    mo = eri
+    for _ in range(4):
+        mo = torch.tensordot(mo, C, dims=([0], [0]))
+    O, V = slice(0, o), slice(o, o + v)
+    at = dict(i=O, j=O, k=O, l=O, a=V, b=V, c=V, d=V)
+    with CCSD(o, v) as c:
+        for _ in range(2):  # the second call runs on the kept scratch
+            c._check(c.lib.mpqc_ccsd_transform_ao(c.ctx, nbf, *[ctypes.c_void_p(t.data_ptr()) for t in (eri, F, Ci, Ca)],
+                                                  L.MEM_DEVICE))
+        for name in ("Gijab", "Gijkl", "Giajb", "Giabc", "Gijka", "Gabcd"):
+            p, q, r, s = (at[x] for x in name[1:])
+            ref = mo[p, r, q, s].permute(0, 2, 1, 3).contiguous()
+            got = torch.empty_like(ref)
+            c._check(c.lib.mpqc_ccsd_get_integral(c.ctx, L.INTEGRAL_IDS[name], ctypes.c_void_p(got.data_ptr()),
+                                                  L.LAYOUT_DENSE, L.MEM_DEVICE))
+            assert float((got - ref).abs().max() / ref.abs().max()) < 1e-12, name

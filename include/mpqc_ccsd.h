@@ -160,7 +160,9 @@ const char* mpqc_ccsd_last_error(const mpqc_ccsd_ctx* ctx);
  * Gijab(l,k,d,c) = Gijab(k,l,c,d); blocks without the symmetry and the adjoint's recorded
  * residual keep the full contractions; 0: the full contractions), "graph" (1 default: the FP64
  * and FP32 residual is captured into a HIP graph on its second call and replayed; any option
- * change or new integrals re-capture; 0: eager launches), "solve_restart" (1 default: solve()
+ * change or new integrals re-capture; 0: eager launches), "levels" (1 default: the FP64 residual of the
+ * standard method with o^2 v^2 <= 2^20 runs its small ops in a few launches of independent ones;
+ * 0: one launch per op), "solve_restart" (1 default: solve()
  * starts from the initial guess; 0: from the context's amplitudes; 2: from them projected onto
  * t2(a,b,i,j) = t2(b,a,j,i)).  Tuning keys that act on
  * every context of the process (measurement aids; the defaults are the measured best):

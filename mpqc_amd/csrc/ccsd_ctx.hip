@@ -213,6 +213,9 @@ void CCSDContext::set_option(const std::string& key, double value) {
   if (key == "graph") {  // 1: replay the FP64/FP32 residual from a HIP graph
     if (value != 0.0 && value != 1.0) throw std::invalid_argument("graph must be 0 or 1");
     graph_mode_ = (int)value;
+  } else if (key == "levels") {  // 1: small FP64 residuals by levels of independent ops
+    if (value != 0.0 && value != 1.0) throw std::invalid_argument("levels must be 0 or 1");
+    levels_mode_ = (int)value;
   } else if (key == "fov_sign") {
     if (value != 1.0 && value != -1.0) throw std::invalid_argument("fov_sign must be +1 or -1");
     fov_sign_ = value;
@@ -1023,6 +1026,7 @@ void CCSDContext::residual() {
     tau_amax_fresh_ = false;
   }
   if (!tape_ || tape_execute_) tau_fresh_ = true;  // (a tape recorded without executing runs nothing)
+  if (levels_usable()) plan_levels();
   if (graph_eligible()) {
     if (res_exec_ && res_graph_gen_ == gen_) {
       MPQC_HIP_CHECK(hipGraphLaunch(res_exec_, stream_));
@@ -1041,6 +1045,10 @@ void CCSDContext::residual() {
 }
 
 void CCSDContext::residual_ops() {
+  if (levels_usable() && levels_gen_ == gen_) {
+    run_levels();
+    return;
+  }
   const int o = o_, v = v_;
   const long O = o, V = v;
   const long ov = O * V, oo = O * O, vv = V * V;

@@ -4,6 +4,7 @@
 
 #include <array>
 #include <deque>
+#include <functional>
 #include <string>
 #include <vector>
 
@@ -357,6 +358,24 @@ class CCSDContext {
   hipGraph_t res_graph_ = nullptr;
   hipGraphExec_t res_exec_ = nullptr;
   bool graph_eligible() const;
+  // ---- small molecules: the residual's ops in a few launches of independent ops
+  // (ccsd_levels.hip); planned once per configuration
+  struct Level {
+    int first_op, nops, groups;  // ops of its launch
+    std::vector<int> calls;      // of level_calls_: large contractions, launched by themselves
+  };
+  std::vector<Level> levels_;
+  std::vector<std::function<void()>> level_calls_;
+  double* levels_ops_ = nullptr;  // device op records
+  size_t levels_ops_n_ = 0;
+  double* levels_ws_ = nullptr;   // partial sums
+  size_t levels_ws_n_ = 0;
+  long levels_gen_ = -1;
+  static constexpr long kLevelMaxDoubles = 1L << 20;  // o^2 v^2
+  int levels_mode_ = 1;           // option "levels"
+  bool levels_usable() const;
+  void plan_levels();
+  void run_levels();
   void residual_ops();
   bool capture_residual();
   void drop_residual_graph();

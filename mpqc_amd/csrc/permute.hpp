@@ -83,21 +83,23 @@ inline int perm_fast_tile(const PermGeom& g) {
 // selects the code compiled in: 0 linear only, 1 tiled only, 2 both (decided by
 // g.tiled), 3 and 4 the fast tile shapes of perm_fast_tile(); kernels launched for one
 // shape keep the other shapes' registers out.
-template <int SHAPE = 2, class Store>
+// THREADS: of the workgroup; lds: perm_lds_bytes(g) of LDS.
+extern __shared__ double perm_tile[];  // dynamic LDS of the launches of one permutation
+template <int SHAPE = 2, int THREADS = kPThreads, class Store>
 __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by, unsigned bz,
-                                     Store&& store) {
+                                     Store&& store, double* lds = perm_tile) {
   if (SHAPE == 0 || (SHAPE == 2 && !g.tiled)) {
     // linear shape: q = 2, r1 = 1, r0 = 0; the host keeps the (q,3) plane below 2^31.
-    // kLinPer elements per thread, kPThreads apart (every access coalesced); all of a
+    // kLinPer elements per thread, THREADS apart (every access coalesced); all of a
     // thread's sums are formed before its stores, so its loads are in flight together.
     const long plane = g.nq * g.n3;
-    const long e0 = (long)bx * (kPThreads * kLinPer) + threadIdx.x;
+    const long e0 = (long)bx * (THREADS * kLinPer) + threadIdx.x;
     const long ir1 = by, ir0 = bz;
     const int n3 = (int)g.n3;
     int iq[kLinPer], i3[kLinPer];  // (elements past the plane read element 0)
 #pragma unroll
     for (int j = 0; j < kLinPer; ++j) {
-      const long ej = e0 + (long)j * kPThreads;
+      const long ej = e0 + (long)j * THREADS;
       const int e = ej < plane ? (int)ej : 0;
       iq[j] = e / n3;
       i3[j] = e - iq[j] * n3;
@@ -121,18 +123,17 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
                   g.py[ir0 * g.pyr0 + ir1 * g.pyr1 + (long)iq[j] * g.pyq + (long)i3[j] * g.py3];
 #pragma unroll
     for (int j = 0; j < kLinPer; ++j) {
-      const long ej = e0 + (long)j * kPThreads;
+      const long ej = e0 + (long)j * THREADS;
       if (ej < plane) store(ir0 * g.or0 + ir1 * g.or1 + ej, acc[j]);
     }
     return;
   }
-  extern __shared__ double perm_tile[];  // T3 x (TQ + 1), perm_lds_bytes()
-  double* tile = perm_tile;
+  double* tile = lds;  // T3 x (TQ + 1)
   const int T3 = g.t3, TQ = g.tq, nel = T3 * TQ, ld = TQ + 1;
   const int t3i = (int)bx % g.tiles3, tqi = (int)bx / g.tiles3;
   const long ir1 = by, ir0 = bz;
   const long b3 = (long)t3i * T3, bq = (long)tqi * TQ;
-  constexpr int kPer = kPTEl / kPThreads;
+  constexpr int kPer = kPTEl / THREADS;
   if (SHAPE == 3 || SHAPE == 4) {
     // perm_fast_tile(): inputs through the tile one after another, the others read along
     // dim 3; each output element sums its terms in term order, then the product term.
@@ -144,7 +145,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
       const int s3 = (int)T.s3;
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        const int e = (int)threadIdx.x + k * kPThreads;
+        const int e = (int)threadIdx.x + k * THREADS;
         if (e < nel) {
           const int jj = (int)(((float)e + 0.5f) * g.inv_tq), qq = e - jj * TQ;
           tile[jj * ld + qq] = (qq < nq && jj < n3) ? src[qq + jj * s3] : 0.0;
@@ -159,7 +160,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
     double v[kPer];
 #pragma unroll
     for (int k = 0; k < kPer; ++k) {
-      const int e = (int)threadIdx.x + k * kPThreads;
+      const int e = (int)threadIdx.x + k * THREADS;
       ql[k] = (int)(((float)e + 0.5f) * g.inv_t3);
       j3[k] = e - ql[k] * T3;
       in[k] = e < nel && ql[k] < nq && j3[k] < n3;
@@ -209,7 +210,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
       // lanes run along q, where this input is contiguous
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        const int e = (int)threadIdx.x + k * kPThreads;
+        const int e = (int)threadIdx.x + k * THREADS;
         if (e < nel) {
           const int j3 = (int)(((float)e + 0.5f) * g.inv_tq), ql = e - j3 * TQ;
           const long iq = bq + ql, i3 = b3 + j3;
@@ -219,7 +220,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
       __syncthreads();
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        const int e = (int)threadIdx.x + k * kPThreads;
+        const int e = (int)threadIdx.x + k * THREADS;
         if (e < nel) {
           const int ql = (int)(((float)e + 0.5f) * g.inv_t3), j3 = e - ql * T3;
           acc[k] += T.alpha * tile[j3 * ld + ql];
@@ -229,7 +230,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
     } else {
 #pragma unroll
       for (int k = 0; k < kPer; ++k) {
-        const int e = (int)threadIdx.x + k * kPThreads;
+        const int e = (int)threadIdx.x + k * THREADS;
         if (e < nel) {
           const int ql = (int)(((float)e + 0.5f) * g.inv_t3), j3 = e - ql * T3;
           const long iq = bq + ql, i3 = b3 + j3;
@@ -240,7 +241,7 @@ __device__ inline void permute_block(const PermGeom& g, unsigned bx, unsigned by
   }
 #pragma unroll
   for (int k = 0; k < kPer; ++k) {
-    const int e = (int)threadIdx.x + k * kPThreads;
+    const int e = (int)threadIdx.x + k * THREADS;
     if (e < nel) {
       const int ql = (int)(((float)e + 0.5f) * g.inv_t3), j3 = e - ql * T3;
       const long iq = bq + ql, i3 = b3 + j3;

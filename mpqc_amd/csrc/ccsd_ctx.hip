@@ -127,6 +127,8 @@ void CCSDContext::release() {
   modeinfo_ = nullptr;
   if (staging_) hipFree(staging_);
   staging_ = nullptr;
+  if (host_scalars_) (void)hipHostFree(host_scalars_);
+  host_scalars_ = nullptr;
   if (stream_) hipStreamDestroy(stream_);
   stream_ = nullptr;
 }
@@ -180,6 +182,7 @@ void CCSDContext::construct(const int64_t* occ_hm, int n_occ_tiles, const int64_
   ws_.bytes = ws_elems * sizeof(double);
   partials_ = alloc(kReducePartials);
   scalars_ = alloc(64);
+  MPQC_HIP_CHECK(hipHostMalloc((void**)&host_scalars_, 64 * sizeof(double), hipHostMallocDefault));
   if (with_solver) solver_init(1, 8, 0.0, 1, 1);
   MPQC_HIP_CHECK(hipMemsetAsync(t1_, 0, ov * sizeof(double), stream_));
   MPQC_HIP_CHECK(hipMemsetAsync(t2_, 0, oovv * sizeof(double), stream_));
@@ -1393,23 +1396,54 @@ void CCSDContext::residual_ops() {
 }
 
 // ---------------------------------------------------------------- energy / error / update
-void CCSDContext::energy_error(double* E, double* err) {
+std::vector<int> CCSDContext::diis_kept(int* slot) const {
+  std::vector<int> kept(err_slots_.begin(), err_slots_.end());
+  if ((int)kept.size() == n_diis_) kept.erase(kept.begin());  // the oldest makes room
+  std::vector<bool> used(n_diis_, false);
+  for (int s : kept) used[s] = true;
+  *slot = 0;
+  while (used[*slot]) ++*slot;
+  return kept;
+}
+
+void CCSDContext::energy_error(double* E, double* err, std::vector<double>* dots) {
   if (!prepared_) prepare();
   const long n1 = (long)o_ * v_, n2 = n1 * n1;
   // error = sqrt(|r1|^2 + |r2|^2) / (size(r1) + size(r2))   qc/cc/solvers.h:60-63
   // E = 2 <f_ai + r1, t1> + <g_abij + r2, 2 tau(a,b,i,j) - tau(b,a,i,j)>   ccsd.h:377-379
   // (with the two norms, in one pass over r2)
-  timed("en:energy", 0.0, [&] {
-    ccsd_energy_norms(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, scalars_, partials_, stream_);
-  });
-  double h[3];
-  MPQC_HIP_CHECK(hipMemcpyAsync(h, scalars_, 3 * sizeof(double), hipMemcpyDeviceToHost, stream_));
+  int nvec = 0;
+  if (dots) {
+    // r goes into the slot that update() would give it: a free one, or that of the oldest
+    // vector, which no later update() reads
+    int slot;
+    const std::vector<int> kept = diis_kept(&slot);
+    nvec = (int)kept.size();
+    std::vector<const double*> x1, x2;
+    for (int s : kept) {
+      x1.push_back(hist_e1_[s]);
+      x2.push_back(hist_e2_[s]);
+    }
+    timed("en:energy_dots", 0.0, [&] {
+      ccsd_energy_dots(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, x1.data(), x2.data(), nvec, hist_e1_[slot],
+                       hist_e2_[slot], host_scalars_, partials_, stream_);
+    });
+  } else {
+    timed("en:energy", 0.0, [&] {
+      ccsd_energy_norms(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, host_scalars_, partials_, stream_);
+    });
+  }
   MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
+  const double* h = host_scalars_;
   const double e = std::sqrt(h[0] + h[1]) / (double)(n1 + n2);
   if (!std::isfinite(e) || !std::isfinite(h[2]))
     throw std::range_error("non-finite residual or energy");
   if (err) *err = e;
   if (E) *E = h[2];
+  if (dots) {
+    dots->assign(h + 3, h + 3 + nvec);
+    dots->push_back(h[0] + h[1]);
+  }
 }
 
 void CCSDContext::check_finite(const double* x, long n, const char* what) {
@@ -1420,13 +1454,15 @@ void CCSDContext::check_finite(const double* x, long n, const char* what) {
 // DIISSolver::update (qc/cc/solvers.h:112-121): Jacobi update_only
 // (lcao/cc/solvers.h:1153-1158), then TA::DIIS::extrapolate(t, r) with the
 // pre-update residuals as error vectors; then tau (ccsd.h:389).
-void CCSDContext::update() {
+void CCSDContext::update(const std::vector<double>* dots) {
   if (!have_eps_) throw std::logic_error("orbital energies not set");
   if (!solver_ready_) throw std::logic_error("solver not initialised");
   const long n1 = (long)o_ * v_, n2 = n1 * n1;
   // --- DIIS: push the error (copy of r) into the history
   ++diis_iter_;
   const double scale = 1.0 + diis_damp_;
+  int eslot = 0;
+  diis_kept(&eslot);
   if ((int)err_slots_.size() == n_diis_) {
     err_slots_.pop_front();
     // drop first row/column of B
@@ -1436,29 +1472,27 @@ void CCSDContext::update() {
       for (int j = 1; j < m; ++j) Bn[(size_t)(i - 1) * m + (j - 1)] = B_[(size_t)i * m + j];
     B_ = Bn;
   }
-  int eslot = 0;
-  {
-    std::vector<bool> used(n_diis_, false);
-    for (int s : err_slots_) used[s] = true;
-    while (used[eslot]) ++eslot;
-  }
   err_slots_.push_back(eslot);
   const int nvec = (int)err_slots_.size();
   {
-    // the new error vector r goes into its slot in the pass that forms its overlaps with
-    // the history (its own overlap read from r itself)
-    std::vector<const double*> x1, x2;
-    for (int s : err_slots_) {
-      x1.push_back(s == eslot ? r1_ : hist_e1_[s]);
-      x2.push_back(s == eslot ? r2_ : hist_e2_[s]);
+    const double* h = host_scalars_ + 32;
+    if (dots) {
+      if ((int)dots->size() != nvec) throw std::logic_error("DIIS: overlaps of another history");
+      h = dots->data();
+    } else {
+      // the new error vector r goes into its slot in the pass that forms its overlaps with
+      // the history (its own overlap read from r itself)
+      std::vector<const double*> x1, x2;
+      for (int s : err_slots_) {
+        x1.push_back(s == eslot ? r1_ : hist_e1_[s]);
+        x2.push_back(s == eslot ? r2_ : hist_e2_[s]);
+      }
+      timed("up:diis_dots", 0.0, [&] {
+        multi_dot2(x1.data(), x2.data(), nvec, r1_, r2_, n1, n2, host_scalars_ + 32, partials_, stream_, hist_e1_[eslot],
+                   hist_e2_[eslot]);
+      });
+      MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
     }
-    timed("up:diis_dots", 0.0, [&] {
-      multi_dot2(x1.data(), x2.data(), nvec, r1_, r2_, n1, n2, scalars_ + 16, partials_, stream_, hist_e1_[eslot],
-                 hist_e2_[eslot]);
-    });
-    double h[16];
-    MPQC_HIP_CHECK(hipMemcpyAsync(h, scalars_ + 16, nvec * sizeof(double), hipMemcpyDeviceToHost, stream_));
-    MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
     const int m = n_diis_;
     for (int i = 0; i < nvec; ++i) B_[(size_t)i * m + (nvec - 1)] = B_[(size_t)(nvec - 1) * m + i] = h[i];
   }
@@ -1470,9 +1504,6 @@ void CCSDContext::update() {
     for (int s : x_slots_) used[s] = true;
     while (used[xslot]) ++xslot;
   }
-  timed("up:jacobi", 0.0, [&] {
-    jacobi_update(t1_, t2_, r1_, r2_, eo_, ev_, o_, v_, stream_, hist_x1_[xslot], hist_x2_[xslot]);
-  });
   x_slots_.push_back(xslot);
   const bool do_extrap =
       diis_iter_ > diis_start_ && ((diis_iter_ - diis_start_) % diis_ngroup_) < diis_group_nstart_;
@@ -1514,21 +1545,25 @@ void CCSDContext::update() {
     }
   }
   // tau("a,b,i,j") = t2 + t1 t1                                     ccsd.h:389
-  // (with the maxima the fp16 splits need; after an extrapolation, in the pass that writes t2)
+  // (with the maxima the fp16 splits need; with an extrapolation, in the pass that makes t2)
   double* maxes = (prec_ == GemmPrecision::F16X3 && amax_.dev) ? amax_.dev + 1 : nullptr;
-  if (do_extrap) {
+  if (do_extrap) {  // the Jacobi step's vector is the last of the history
     timed("up:extrapolate", 0.0, [&] {
-      lincomb(t1_, x1.data(), c.data(), (int)c.size(), n1, stream_);
-      lincomb_tau(t2_, tau_, t1_, x2.data(), c.data(), (int)c.size(), o_, v_, partials_, maxes, stream_);
+      jacobi_extrapolate(t1_, t2_, tau_, r1_, r2_, eo_, ev_, o_, v_, hist_x1_[xslot], hist_x2_[xslot], x1.data(),
+                         x2.data(), c.data(), (int)c.size() - 1, c.back(), partials_, maxes, stream_);
     });
-  } else if (maxes) {
-    timed("up:tau", 0.0, [&] { build_tau_absmax(tau_, t2_, t1_, o_, v_, partials_, maxes, stream_); });
   } else {
-    timed("up:tau", 0.0, [&] { build_tau(tau_, t2_, t1_, o_, v_, stream_); });
+    timed("up:jacobi", 0.0, [&] {
+      jacobi_update(t1_, t2_, r1_, r2_, eo_, ev_, o_, v_, stream_, hist_x1_[xslot], hist_x2_[xslot]);
+    });
+    timed("up:tau", 0.0, [&] {
+      if (maxes) build_tau_absmax(tau_, t2_, t1_, o_, v_, partials_, maxes, stream_);
+      else build_tau(tau_, t2_, t1_, o_, v_, stream_);
+    });
   }
   tau_amax_fresh_ = maxes != nullptr;
   tau_fresh_ = true;
-  MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
+  if (!dots) MPQC_HIP_CHECK(hipStreamSynchronize(stream_));  // (the solver loop queues the residual behind it)
 }
 
 // CCSD::compute_ccsd solver loop (ccsd.h:344-477) with method = "standard".
@@ -1550,14 +1585,15 @@ double CCSDContext::solve(int max_iter, double target_precision, int verbose, in
   trace_.clear();
   double E0 = 0.0, E1 = 0.0, dE = 0.0, err = 1.0;
   int iter = 0;
+  std::vector<double> dots;
   auto t0 = std::chrono::steady_clock::now();
   while (iter < max_iter) {
-    energy_error(&E1, &err);  // error (:373) and energy (:377-379); E1 uses t of this pass
+    energy_error(&E1, &err, &dots);  // error (:373) and energy (:377-379); E1 uses t of this pass
     dE = std::fabs(E0 - E1);
     E0 = E1;
     const bool converged = dE <= target_precision * 0.1 && err <= target_precision;  // :141-152
     if (iter == 0 || !converged) {
-      update();
+      update(&dots);
       auto t1 = std::chrono::steady_clock::now();
       if (iter > 0) {
         const double sec = std::chrono::duration<double>(t1 - t0).count();

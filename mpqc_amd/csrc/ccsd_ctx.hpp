@@ -74,8 +74,10 @@ class CCSDContext {
 
   void init_guess();
   void residual();
-  void energy_error(double* E, double* err);
-  void update();
+  // with dots: also the overlaps of the residual with the DIIS history that update(dots) pushes
+  // it onto (the newest last), from the same pass
+  void energy_error(double* E, double* err, std::vector<double>* dots = nullptr);
+  void update(const std::vector<double>* dots = nullptr);
   double solve(int max_iter, double target_precision, int verbose, int* n_iter);
   const std::vector<TraceRow>& trace() const { return trace_; }
   // (T) correction from the current (converged) amplitudes (CCSD_T::compute_ccsd_t,
@@ -331,6 +333,10 @@ class CCSDContext {
   GemmWorkspace ws_;
   double* partials_ = nullptr;
   double* scalars_ = nullptr;  // device scalars
+  // pinned host memory that the last pass of a reduction writes (no copy back to wait for)
+  double* host_scalars_ = nullptr;
+  // DIIS error vectors that stay when one is pushed, and the slot the new one takes
+  std::vector<int> diis_kept(int* slot) const;
   long* modeinfo_ = nullptr;   // device tile maps (scratch, sized per call)
   size_t modeinfo_n_ = 0;
   double* staging_ = nullptr;  // device staging for tiled / host uploads

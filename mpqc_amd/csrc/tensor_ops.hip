@@ -291,6 +291,68 @@ __global__ __launch_bounds__(kBlock) void multidot_vec_stage1(MultiDotArgs a, do
   }
 }
 
+// One pass over the residuals for a solver step: the sums of energy_norms_stage1 and the
+// overlaps of r with the DIIS history (r itself also written into its history slot):
+// partials[k * gridDim.x + block], k = 0 |r1|^2, 1 |r2|^2, 2 energy, 3 + q <x_q, r>.  W = 2:
+// two elements per 16-byte access (o^2 even, so a pair has one (a,b); arrays aligned).
+// Bound: HBM, (nvec + 5) o^2 v^2 doubles; the separate passes read r2 twice and cost a second
+// round trip to the host ((H2O)8: 404 us against 203 + 224 us; at the water molecule's sizes,
+// where a round trip costs more than any kernel, an iteration went from 217 to 150 us with the
+// two fusions below and the sums written to host memory).
+template <int W>
+__global__ __launch_bounds__(kBlock) void energy_dots_stage1(MultiDotArgs a, const double* __restrict__ f_ai,
+                                                             const double* __restrict__ t1,
+                                                             const double* __restrict__ g,
+                                                             const double* __restrict__ tau, int o, int v,
+                                                             double* __restrict__ partials) {
+  typedef double vec_t __attribute__((ext_vector_type(W)));
+  constexpr int kMaxHist = 15;
+  const int oo = o * o / W, n2 = v * v * oo;
+  const vec_t* __restrict__ g2 = reinterpret_cast<const vec_t*>(g);
+  const vec_t* __restrict__ tau2 = reinterpret_cast<const vec_t*>(tau);
+  const vec_t* __restrict__ r2 = reinterpret_cast<const vec_t*>(a.y2);
+  double acc[kMaxHist], e2 = 0.0, q2 = 0.0, e1 = 0.0, q1 = 0.0;
+#pragma unroll
+  for (int k = 0; k < kMaxHist; ++k) acc[k] = 0.0;
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < n2; e += gridDim.x * kBlock) {
+    const int ab = e / oo, ij = e - ab * oo;
+    const int ai = ab / v, bi = ab - ai * v;
+    const vec_t r = r2[e], gg = g2[e], t = tau2[e], tx = tau2[(bi * v + ai) * oo + ij];
+    reinterpret_cast<vec_t*>(a.c2)[e] = r;
+#pragma unroll
+    for (int w = 0; w < W; ++w) {
+      e2 += (gg[w] + r[w]) * (2.0 * t[w] - tx[w]);
+      q2 += r[w] * r[w];
+    }
+#pragma unroll
+    for (int k = 0; k < kMaxHist; ++k)
+      if (k < a.nvec) {
+        const vec_t x = reinterpret_cast<const vec_t*>(a.x2[k])[e];
+#pragma unroll
+        for (int w = 0; w < W; ++w) acc[k] += x[w] * r[w];
+      }
+  }
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < v * o; e += gridDim.x * kBlock) {
+    const double r = a.y1[e];
+    a.c1[e] = r;
+    e1 += (f_ai[e] + r) * t1[e];
+    q1 += r * r;
+#pragma unroll
+    for (int k = 0; k < kMaxHist; ++k)
+      if (k < a.nvec) acc[k] += a.x1[k][e] * r;
+  }
+  const double s1 = block_sum(q1), s2 = block_sum(q2), se = block_sum(e2 + 2.0 * e1);
+  if (threadIdx.x == 0) {
+    partials[blockIdx.x] = s1;
+    partials[gridDim.x + blockIdx.x] = s2;
+    partials[2 * gridDim.x + blockIdx.x] = se;
+  }
+  for (int k = 0; k < a.nvec; ++k) {
+    const double r = block_sum(acc[k]);
+    if (threadIdx.x == 0) partials[(long)(3 + k) * gridDim.x + blockIdx.x] = r;
+  }
+}
+
 struct LincombArgs {
   const double* x[16];
   double c[16];
@@ -320,25 +382,52 @@ __global__ __launch_bounds__(kBlock) void lincomb_kernel(double* __restrict__ y,
   }
 }
 
-// t2 = sum_k c_k x_k (lincomb_kernel's sum) and tau = t2 + t1(a,i) t1(b,j) (build_tau's)
-// in one pass; with part, also the per-block max |t2| and max |tau| (build_tau_absmax's).
+// Jacobi step and extrapolation of t1: x = t1 + r1 / D into its history slot,
+// t1 = sum_k c_k x_k + cx x.
+__global__ __launch_bounds__(kBlock) void jacobi_extrapolate1_kernel(double* __restrict__ t1,
+                                                                     const double* __restrict__ r1,
+                                                                     const double* __restrict__ eo,
+                                                                     const double* __restrict__ ev, int o, int v,
+                                                                     double* __restrict__ slot, LincombArgs a,
+                                                                     double cx) {
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < v * o; e += gridDim.x * kBlock) {
+    const int ai = e / o, i = e - ai * o;
+    const double x = t1[e] + r1[e] / (eo[i] - ev[ai]);
+    slot[e] = x;
+    double acc = 0.0;
+    for (int k = 0; k < a.nvec; ++k) acc += a.c[k] * a.x[k][e];
+    t1[e] = acc + cx * x;
+  }
+}
+
+// The same for t2, and tau from the extrapolated t1 and t2 (with MAXES the per-block max
+// |t2| and max |tau| as build_tau_absmax's), in one pass: separate Jacobi and
+// extrapolation passes write and read t2 and the new history vector once more ((H2O)8: 445 us
+// against 253 + 320 us; bound by HBM, (nvec + 5) o^2 v^2 doubles).
 template <bool MAXES>
-__global__ __launch_bounds__(kBlock) void lincomb_tau_kernel(double* __restrict__ t2, double* __restrict__ tau,
-                                                             const double* __restrict__ t1, LincombArgs a, int o,
-                                                             int v, double* __restrict__ part) {
+__global__ __launch_bounds__(kBlock) void jacobi_extrapolate2_kernel(double* __restrict__ t2, double* __restrict__ tau,
+                                                                     const double* __restrict__ t1,
+                                                                     const double* __restrict__ r2,
+                                                                     const double* __restrict__ eo,
+                                                                     const double* __restrict__ ev, int o, int v,
+                                                                     double* __restrict__ slot, LincombArgs a,
+                                                                     double cx, double* __restrict__ part) {
   const int oo = o * o, n = v * v * oo;
   double m2 = 0.0, mt = 0.0;
   for (int e = blockIdx.x * kBlock + threadIdx.x; e < n; e += gridDim.x * kBlock) {
-    double x = 0.0;
-    for (int k = 0; k < a.nvec; ++k) x += a.c[k] * a.x[k][e];
     const int ab = e / oo, ij = e - ab * oo;
     const int ai = ab / v, bi = ab - ai * v;
     const int i = ij / o, j = ij - i * o;
-    const double y = x + t1[ai * o + i] * t1[bi * o + j];
-    t2[e] = x;
+    const double x = t2[e] + r2[e] / (eo[i] + eo[j] - ev[ai] - ev[bi]);
+    slot[e] = x;
+    double acc = 0.0;
+    for (int k = 0; k < a.nvec; ++k) acc += a.c[k] * a.x[k][e];
+    acc += cx * x;
+    const double y = acc + t1[ai * o + i] * t1[bi * o + j];
+    t2[e] = acc;
     tau[e] = y;
     if (MAXES) {
-      m2 = fmax(m2, fabs(x));
+      m2 = fmax(m2, fabs(acc));
       mt = fmax(mt, fabs(y));
     }
   }
@@ -904,24 +993,55 @@ void lincomb(double* y, const double* const* xs, const double* c, int nvec, long
   check_launch("lincomb");
 }
 
-void lincomb_tau(double* t2, double* tau, const double* t1, const double* const* xs, const double* c, int nvec,
-                 int o, int v, double* partials, double* maxes, hipStream_t s) {
+void ccsd_energy_dots(const double* f_ai, const double* r1, const double* t1, const double* g_abij, const double* r2,
+                      const double* tau, int o, int v, const double* const* xs1, const double* const* xs2, int nvec,
+                      double* copy1, double* copy2, double* out, double* partials, hipStream_t s) {
   check_small(o, v);
-  if (nvec > 16) throw std::invalid_argument("lincomb: at most 16 vectors");
-  LincombArgs a;
+  if (nvec > 15) throw std::invalid_argument("ccsd_energy_dots: at most 15 vectors");
+  MultiDotArgs a;
   for (int k = 0; k < 16; ++k) {
-    a.x[k] = k < nvec ? xs[k] : nullptr;
-    a.c[k] = k < nvec ? c[k] : 0.0;
+    a.x1[k] = k < nvec ? xs1[k] : nullptr;
+    a.x2[k] = k < nvec ? xs2[k] : nullptr;
   }
-  a.nvec = nvec;
+  a.y1 = r1; a.y2 = r2; a.c1 = copy1; a.c2 = copy2; a.nvec = nvec;
+  a.n1 = (long)v * o; a.n2 = a.n1 * a.n1;
+  auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  bool vec = o % 2 == 0 && a.n2 >= 2 * (long)kBlock * kRedGrid && al16(r2) && al16(copy2) && al16(g_abij) && al16(tau);
+  for (int k = 0; k < nvec; ++k) vec = vec && al16(xs2[k]);
+  const int g = red_grid(vec ? a.n2 / 2 : a.n2);
+  if (vec)
+    hipLaunchKernelGGL(energy_dots_stage1<2>, dim3(g), dim3(kBlock), 0, s, a, f_ai, t1, g_abij, tau, o, v, partials);
+  else
+    hipLaunchKernelGGL(energy_dots_stage1<1>, dim3(g), dim3(kBlock), 0, s, a, f_ai, t1, g_abij, tau, o, v, partials);
+  hipLaunchKernelGGL(reduce_stage2, dim3(3 + nvec), dim3(kBlock), 0, s, partials, g, out, 1.0);
+  check_launch("ccsd_energy_dots");
+}
+
+void jacobi_extrapolate(double* t1, double* t2, double* tau, const double* r1, const double* r2, const double* eps_o,
+                        const double* eps_v, int o, int v, double* slot1, double* slot2, const double* const* xs1,
+                        const double* const* xs2, const double* c, int nvec, double cx, double* partials,
+                        double* maxes, hipStream_t s) {
+  check_small(o, v);
+  if (nvec > 15) throw std::invalid_argument("jacobi_extrapolate: at most 15 older vectors");
+  LincombArgs a1, a2;
+  for (int k = 0; k < 16; ++k) {
+    a1.x[k] = k < nvec ? xs1[k] : nullptr;
+    a2.x[k] = k < nvec ? xs2[k] : nullptr;
+    a1.c[k] = a2.c[k] = k < nvec ? c[k] : 0.0;
+  }
+  a1.nvec = a2.nvec = nvec;
+  hipLaunchKernelGGL(jacobi_extrapolate1_kernel, dim3(elem_grid((long)v * o)), dim3(kBlock), 0, s, t1, r1, eps_o, eps_v,
+                     o, v, slot1, a1, cx);
   const int nb = (int)std::min<long>(elem_grid((long)v * v * o * o), kReducePartials / 2);
   if (maxes) {
-    hipLaunchKernelGGL(lincomb_tau_kernel<true>, dim3(nb), dim3(kBlock), 0, s, t2, tau, t1, a, o, v, partials);
+    hipLaunchKernelGGL(jacobi_extrapolate2_kernel<true>, dim3(nb), dim3(kBlock), 0, s, t2, tau, t1, r2, eps_o, eps_v, o,
+                       v, slot2, a2, cx, partials);
     hipLaunchKernelGGL(absmax2_stage2, dim3(1), dim3(kBlock), 0, s, partials, nb, maxes);
   } else {
-    hipLaunchKernelGGL(lincomb_tau_kernel<false>, dim3(nb), dim3(kBlock), 0, s, t2, tau, t1, a, o, v, partials);
+    hipLaunchKernelGGL(jacobi_extrapolate2_kernel<false>, dim3(nb), dim3(kBlock), 0, s, t2, tau, t1, r2, eps_o, eps_v,
+                       o, v, slot2, a2, cx, partials);
   }
-  check_launch("lincomb_tau");
+  check_launch("jacobi_extrapolate");
 }
 
 void count_nonfinite(const double* x, long n, double* out, double* partials, hipStream_t s) {

@@ -96,11 +96,19 @@ void fill(double* x, long n, double value, hipStream_t s);
 
 // y = sum_k c_k x_k, k < nvec (fixed summation order)
 void lincomb(double* y, const double* const* xs, const double* c, int nvec, long n, hipStream_t s);
-// t2 = sum_k c[k] xs[k] (as lincomb) and tau = t2 + t1(a,i) t1(b,j) (as build_tau) in one
-// pass over the o^2 v^2 elements; with maxes, also max |t2| and max |tau| into maxes[0..1]
-// (as build_tau_absmax).
-void lincomb_tau(double* t2, double* tau, const double* t1, const double* const* xs, const double* c, int nvec,
-                 int o, int v, double* partials, double* maxes, hipStream_t s);
+// A solver step's sums in one pass over r: out[0] = |r1|^2, out[1] = |r2|^2, out[2] the energy
+// (as ccsd_energy_norms), out[3 + k] = <x_k, r> for nvec <= 15 history vectors; r is copied
+// to (copy1, copy2).
+void ccsd_energy_dots(const double* f_ai, const double* r1, const double* t1, const double* g_abij, const double* r2,
+                      const double* tau, int o, int v, const double* const* xs1, const double* const* xs2, int nvec,
+                      double* copy1, double* copy2, double* out, double* partials, hipStream_t s);
+// Jacobi step, its history copy, extrapolation and tau in one pass over t2:
+// slot = t + r / D, t = sum_k c[k] xs[k] + cx slot, tau = t2 + t1(a,i) t1(b,j); with maxes also max |t2|
+// and max |tau| into maxes[0..1] (as build_tau_absmax).
+void jacobi_extrapolate(double* t1, double* t2, double* tau, const double* r1, const double* r2, const double* eps_o,
+                        const double* eps_v, int o, int v, double* slot1, double* slot2, const double* const* xs1,
+                        const double* const* xs2, const double* c, int nvec, double cx, double* partials,
+                        double* maxes, hipStream_t s);
 
 // Number of doubles of `partials` scratch the reductions above need.
 constexpr long kReducePartials = 4096 * 16;

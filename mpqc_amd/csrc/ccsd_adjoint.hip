@@ -319,11 +319,9 @@ void CCSDContext::jacobian_transpose_io(const double* y1, const double* y2, doub
   double* dy2 = adj_hist(101, n2);
   double* dx1 = adj_hist(102, n1);
   double* dx2 = adj_hist(103, n2);
-  upload(dy1, y1, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  upload(dy2, y2, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+  upload_pair(dy1, dy2, y1, y2, false, layout, memspace);
   jacobian_transpose(dy1, dy2, dx1, dx2);
-  download(x1, dx1, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  download(x2, dx2, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+  download_pair(x1, x2, dx1, dx2, layout, memspace);
 }
 
 // Lambda equations (dR/dt)^T lambda = -dE/dt, solved with the amplitude
@@ -482,8 +480,7 @@ void CCSDContext::energy_gradient() {
 
 void CCSDContext::get_lambda(double* l1, double* l2, int layout, int memspace) {
   if (!lambda_ready_) throw std::logic_error("solve the Lambda equations first");
-  if (l1) download(l1, lam1_, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  if (l2) download(l2, lam2_, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+  download_pair(l1, l2, lam1_, lam2_, layout, memspace);
 }
 
 void CCSDContext::get_integral_gradient(int which, double* out, int layout, int memspace) {

@@ -182,6 +182,7 @@ void CCSDContext::construct(const int64_t* occ_hm, int n_occ_tiles, const int64_
   ws_.bytes = ws_elems * sizeof(double);
   partials_ = alloc(kReducePartials);
   scalars_ = alloc(64);
+  MPQC_HIP_CHECK(hipGetDevice(&device_));
   MPQC_HIP_CHECK(hipHostMalloc((void**)&host_scalars_, 64 * sizeof(double), hipHostMallocDefault));
   if (with_solver) solver_init(1, 8, 0.0, 1, 1);
   MPQC_HIP_CHECK(hipMemsetAsync(t1_, 0, ov * sizeof(double), stream_));
@@ -500,23 +501,69 @@ void CCSDContext::solver_init(int diis_start, int n_diis, double damp, int ngrou
   solver_ready_ = true;
 }
 
-void CCSDContext::set_amplitudes(const double* t1, const double* t2, int layout, int memspace) {
-  upload(t1_, t1, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  upload(t2_, t2, {kVir, kVir, kOcc, kOcc}, layout, memspace);
-  build_tau(tau_, t2_, t1_, o_, v_, stream_);
-  tau_fresh_ = true;
-  tau_amax_fresh_ = false;
+// Whether p[0..n) is a dense array that a kernel on this context's device may access: inside
+// one allocation of that device (what hipMemcpy checks of its arguments), doubles aligned.
+bool CCSDContext::device_array(const double* p, long n) const {
+  hipPointerAttribute_t at{};
+  if (reinterpret_cast<uintptr_t>(p) % sizeof(double) || hipPointerGetAttributes(&at, p) != hipSuccess ||
+      at.type != hipMemoryTypeDevice || at.device != device_) {
+    (void)hipGetLastError();
+    return false;
+  }
+  hipDeviceptr_t base = nullptr;
+  size_t size = 0;
+  if (hipMemGetAddressRange(&base, &size, const_cast<double*>(p)) != hipSuccess) {
+    (void)hipGetLastError();
+    return false;
+  }
+  return (size_t)((const char*)p - (const char*)base) + n * sizeof(double) <= size;
+}
+
+// (above it copy_pair's 32-bit indices could pass 2^31, and its gain is lost in the transfer)
+constexpr long kPairCopyMax = 1L << 30;
+
+// A (t1, t2)-shaped pair from the caller, with tau_ built from it if asked for.  Dense device
+// arrays take one wait for the caller's pending work, one kernel and one wait for it: two
+// copies and the pass for tau, each with waits of its own, took longer than their transfers
+// (copy_pair's comment).
+void CCSDContext::upload_pair(double* d1, double* d2, const double* s1, const double* s2, bool tau, int layout,
+                              int memspace) {
+  const long n1 = (long)o_ * v_, n2 = n1 * n1;
+  if (layout == 0 && memspace == 1 && n2 <= kPairCopyMax && device_array(s1, n1) && device_array(s2, n2)) {
+    MPQC_HIP_CHECK(hipDeviceSynchronize());  // the caller's pending work on its buffers (as in upload)
+    copy_pair(d1, s1, d2, s2, tau ? tau_ : nullptr, o_, v_, stream_);
+  } else {
+    upload(d1, s1, {kNone, kNone, kVir, kOcc}, layout, memspace);
+    upload(d2, s2, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+    if (tau) build_tau(tau_, d2, d1, o_, v_, stream_);
+  }
   MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
 }
 
+void CCSDContext::download_pair(double* d1, double* d2, const double* s1, const double* s2, int layout, int memspace) {
+  const long n1 = (long)o_ * v_, n2 = n1 * n1;
+  if (d1 && d2 && layout == 0 && memspace == 1 && n2 <= kPairCopyMax && device_array(d1, n1) && device_array(d2, n2)) {
+    MPQC_HIP_CHECK(hipDeviceSynchronize());
+    copy_pair(d1, s1, d2, s2, nullptr, o_, v_, stream_);
+    MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
+    return;
+  }
+  if (d1) download(d1, s1, {kNone, kNone, kVir, kOcc}, layout, memspace);
+  if (d2) download(d2, s2, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+}
+
+void CCSDContext::set_amplitudes(const double* t1, const double* t2, int layout, int memspace) {
+  upload_pair(t1_, t2_, t1, t2, true, layout, memspace);
+  tau_fresh_ = true;
+  tau_amax_fresh_ = false;
+}
+
 void CCSDContext::get_amplitudes(double* t1, double* t2, int layout, int memspace) {
-  if (t1) download(t1, t1_, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  if (t2) download(t2, t2_, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+  download_pair(t1, t2, t1_, t2_, layout, memspace);
 }
 
 void CCSDContext::get_residuals(double* r1, double* r2, int layout, int memspace) {
-  if (r1) download(r1, r1_, {kNone, kNone, kVir, kOcc}, layout, memspace);
-  if (r2) download(r2, r2_, {kVir, kVir, kOcc, kOcc}, layout, memspace);
+  download_pair(r1, r2, r1_, r2_, layout, memspace);
 }
 
 void CCSDContext::get_dressed_fock(double* FIJ, double* FAB) {

@@ -136,6 +136,9 @@ class CCSDContext {
               int memspace);
   void download(double* dst, const double* src, const std::array<int, 4>& modes, int layout,
                 int memspace);
+  bool device_array(const double* p, long n) const;
+  void upload_pair(double* d1, double* d2, const double* s1, const double* s2, bool tau, int layout, int memspace);
+  void download_pair(double* d1, double* d2, const double* s1, const double* s2, int layout, int memspace);
   double* alloc(size_t n);
   // Host-side guard: throws unless [p, p + max_off] lies inside one of this
   // context's device allocations.  Every GEMM and permutation the residual
@@ -332,6 +335,7 @@ class CCSDContext {
       *Xjk_, *Y1_, *Y2_, *RR_, *tmpR_, *Y23_, *W_, *tmp24_;
   GemmWorkspace ws_;
   double* partials_ = nullptr;
+  int device_ = 0;             // the device current at construction, which holds everything
   double* scalars_ = nullptr;  // device scalars
   // pinned host memory that the last pass of a reduction writes (no copy back to wait for)
   double* host_scalars_ = nullptr;

@@ -37,6 +37,32 @@ __global__ __launch_bounds__(kBlock) void build_tau_kernel(double* __restrict__ 
   }
 }
 
+// Both parts of an amplitude-shaped pair in one launch, d1 = s1 and d2 = s2; with TAU also
+// tau = s2 + s1(a,i) s1(b,j).  W = 2: 16-byte accesses (o even, so that a pair has one (a,b);
+// arrays aligned).  Bound: HBM, 2 (3 with tau) o^2 v^2 doubles; two copies and a pass for tau,
+// each waited for, took 40 us more over a residual's set and get at o = 10, v = 90 (890 -> 851 us
+// with the residual) and 540 us more over those of 16 hydrogen chains (10.60 -> 10.06 ms).
+template <int W, bool TAU>
+__global__ __launch_bounds__(kBlock) void copy_pair_kernel(double* __restrict__ d1, const double* __restrict__ s1,
+                                                           double* __restrict__ d2, const double* __restrict__ s2,
+                                                           double* __restrict__ tau, int o, int v) {
+  typedef double vec_t __attribute__((ext_vector_type(W)));
+  const int oo = o * o / W, n = v * v * oo;
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < n; e += gridDim.x * kBlock) {
+    vec_t x = reinterpret_cast<const vec_t*>(s2)[e];
+    reinterpret_cast<vec_t*>(d2)[e] = x;
+    if (TAU) {
+      const int ab = e / oo, ij = (e - ab * oo) * W;
+      const int a = ab / v, b = ab - a * v;
+      const int i = ij / o, j = ij - i * o;
+#pragma unroll
+      for (int w = 0; w < W; ++w) x[w] += s1[a * o + i] * s1[b * o + j + w];
+      reinterpret_cast<vec_t*>(tau)[e] = x;
+    }
+  }
+  for (int e = blockIdx.x * kBlock + threadIdx.x; e < v * o; e += gridDim.x * kBlock) d1[e] = s1[e];
+}
+
 // tau as above, and per block max |t2| and max |tau| -> part[2 blk], part[2 blk + 1]
 __global__ __launch_bounds__(kBlock) void build_tau_absmax_kernel(double* __restrict__ tau,
                                                                   const double* __restrict__ t2,
@@ -815,6 +841,22 @@ void build_tau(double* tau, const double* t2, const double* t1, int o, int v, hi
   hipLaunchKernelGGL(build_tau_kernel, dim3(elem_grid((long)v * v * o * o)), dim3(kBlock), 0, s, tau,
                      t2, t1, o, v);
   check_launch("build_tau");
+}
+
+void copy_pair(double* d1, const double* s1, double* d2, const double* s2, double* tau, int o, int v, hipStream_t s) {
+  check_small(o, v);
+  auto al16 = [](const void* p) { return reinterpret_cast<uintptr_t>(p) % 16 == 0; };
+  const bool vec = o % 2 == 0 && al16(d2) && al16(s2) && (!tau || al16(tau));
+  const dim3 grid(elem_grid((long)v * v * o * o / (vec ? 2 : 1)));
+  auto run = [&](auto kernel) { hipLaunchKernelGGL(kernel, grid, dim3(kBlock), 0, s, d1, s1, d2, s2, tau, o, v); };
+  if (tau) {
+    if (vec) run(copy_pair_kernel<2, true>);
+    else run(copy_pair_kernel<1, true>);
+  } else {
+    if (vec) run(copy_pair_kernel<2, false>);
+    else run(copy_pair_kernel<1, false>);
+  }
+  check_launch("copy_pair");
 }
 
 void build_tau_absmax(double* tau, const double* t2, const double* t1, int o, int v, double* partials,

@@ -45,6 +45,8 @@ void permuted_strides(const long in_extents[4], const int perm[4], long out_s[4]
 
 // tau(a,b,i,j) = t2(a,b,i,j) + t1(a,i) t1(b,j)                 (ccsd.h:389)
 void build_tau(double* tau, const double* t2, const double* t1, int o, int v, hipStream_t s);
+// d1(a,i) = s1, d2(a,b,i,j) = s2 in one launch; with tau also tau = s2 + s1(a,i) s1(b,j)
+void copy_pair(double* d1, const double* s1, double* d2, const double* s2, double* tau, int o, int v, hipStream_t s);
 // build_tau, and maxes[0] = max |t2|, maxes[1] = max |tau| (the fp16 plane scales of the
 // next residual's t2 and tau operands)
 void build_tau_absmax(double* tau, const double* t2, const double* t1, int o, int v, double* partials,

@@ -112,6 +112,7 @@ void CCSDContext::release() {
   event_pool_.clear();
   for (double* p : adj_) if (p) hipFree(p);
   adj_.clear();
+  adj_zero_.clear();
   if (adj_ws_) hipFree(adj_ws_);
   adj_ws_ = nullptr;
   adj_ws_n_ = 0;

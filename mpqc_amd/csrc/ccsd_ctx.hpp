@@ -205,6 +205,7 @@ class CCSDContext {
   };
   // adjoint state
   std::vector<double*> adj_;      // adjoint buffer of allocation k (nullptr until used)
+  std::vector<char> adj_zero_;    // whether that buffer stands for zeros, whatever it holds
   std::vector<TapeOp> res_tape_;  // residual recorded at the amplitudes of the last sweep
   double *lam1_ = nullptr, *lam2_ = nullptr, *gt1_ = nullptr, *gt2_ = nullptr;
   double* adj_ws_ = nullptr;      // partial sums of shared-operand contraction adjoints
@@ -217,7 +218,11 @@ class CCSDContext {
   bool lambda_ready_ = false, gradient_ready_ = false;
   bool lambda_symmetric_ = true;  // solve in the (ab)(ij)-symmetric t2 subspace
   int alloc_index(const double* p) const;
+  int adj_index(const double* p);
   double* adj(const double* p);
+  double* adj_add(const double* p, long n, double* beta);
+  void adj_clear(const double* p, long n);
+  void adj_set(const double* p, const double* src, long n);
   bool is_integral(const double* p) const;
   void zero_adjoints();
   void record_residual();

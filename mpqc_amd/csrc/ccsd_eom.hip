@@ -155,8 +155,8 @@ void CCSDContext::ensure_abcd_from_factors() {
 void CCSDContext::eom_apply_jt(const double* y, double* x) {
   const long O = o_, V = v_, n1 = O * V, n2 = n1 * n1;
   zero_adjoints();
-  MPQC_HIP_CHECK(hipMemcpyAsync(adj(r1_), y, n1 * sizeof(double), hipMemcpyDeviceToDevice, stream_));
-  MPQC_HIP_CHECK(hipMemcpyAsync(adj(r2_), y + n1, n2 * sizeof(double), hipMemcpyDeviceToDevice, stream_));
+  adj_set(r1_, y, n1);
+  adj_set(r2_, y + n1, n2);
   reverse_sweep(res_tape_, false);
   MPQC_HIP_CHECK(hipMemcpyAsync(x, adj(t1_), n1 * sizeof(double), hipMemcpyDeviceToDevice, stream_));
   // x2 = (t2^ + t2^(b,a,j,i)) / 2

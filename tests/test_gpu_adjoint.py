@@ -179,3 +179,27 @@ def test_full_space_gradients_match_arbitrary_perturbations(name):
     an = float(np.vdot(g, X))
     print(f"{name} ({n} Lambda iterations): adjoint {an:.10e} central difference {fd:.10e}")
     assert abs(an - fd) <= 1e-6 * abs(fd)
+
+
+# adjoint buffers hold no stored zeros between sweeps: products that follow others (and a
+# gradient, which also fills the integrals' adjoints) are the same bits as the first one
+@pytest.mark.parametrize("no,nv", [(1, 1), (2, 5), (5, 12), (8, 30)])
+def test_products_repeat_bitwise(no, nv):
+    from mpqc_amd.ccsd import CCSD, Integrals
+    f, b = _random_case(no, nv, seed=no + nv)
+    rng = np.random.default_rng(no * nv)
+    ys = [(rng.normal(0, 1, (nv, no)), rng.normal(0, 1, (nv, nv, no, no))) for _ in range(2)]
+    with CCSD(no, nv, max_iter=40) as c:
+        c.set_integrals(Integrals(**b))
+        c.set_orbital_energies(np.diag(f)[:no], np.diag(f)[no:])
+        c.compute_ccsd(target_precision=1e-10)
+        first = [c.jacobian_transpose(*y) for y in ys]
+        c.lambda_solve()
+        grad = c.energy_gradient()
+        again = [c.jacobian_transpose(*y) for y in reversed(ys)][::-1]
+        c.lambda_solve()
+        grad2 = c.energy_gradient()
+    for p, q in zip(first, again):
+        assert np.array_equal(p[0], q[0]) and np.array_equal(p[1], q[1])
+    for name in grad:
+        assert np.array_equal(grad[name], grad2[name]), name

@@ -276,7 +276,11 @@ void CCSDContext::reverse_op(const TapeOp& op, bool integrals) {
         }
         run(d, g.A, g.lda, g.sA);
       }
-      if (!skip(g.B)) {
+      if (g.A == Gabcd_ && g.B == tau_ && op.tag == "r2:pp_ladder" && tape_pairs()) {
+        double beta;
+        double* bbar = adj_add(g.B, (long)g.K * g.N, &beta);
+        pp_ladder_transposed(cbar, bbar, beta != 0.0, op.prec);
+      } else if (!skip(g.B)) {
         GemmDesc d;
         if (!g.transB) {  // B^(K x N) += a op(A)^T(K x M) C^(M x N)
           d = make_gemm(!g.transA, false, g.K, g.N, g.M, g.alpha, g.A, g.lda, cbar, g.ldc, 1.0, nullptr, 0);

@@ -1433,12 +1433,22 @@ void CCSDContext::residual_ops() {
       df_pp_ladder();  // df :497-508
       return;
     }
-    // :275 b(a,b,i,j) = tau(c,d,i,j) Gabcd(a,b,c,d)  -- the particle-particle ladder (the
-    // recorded residual of the adjoint keeps the full contraction)
+    // :275 b(a,b,i,j) = tau(c,d,i,j) Gabcd(a,b,c,d)  -- the particle-particle ladder (a tape
+    // records the full contraction, run and reversed on pairs where tape_pairs() says so)
+    std::vector<TapeOp>* const tape = tape_;
+    const bool pairs = tape && tape_execute_ && !df_ && tape_pairs();
+    if (pairs) tape_execute_ = false;
     if (psym)
       pp_ladder_symmetric(r2_);
     else
       gemm(false, false, v * v, o * o, v * v, 1.0, Gabcd_, vv, tau_, oo, 1.0, r2_, oo, 0, 0, 0, 1, "r2:pp_ladder");
+    if (pairs) {
+      tape_execute_ = true;
+      tape_ = nullptr;
+      pack_tau_pairs();
+      pp_ladder_symmetric(r2_);
+      tape_ = tape;
+    }
   }
   // (the ladder's T1 terms, :277-280, went into Rd above)
 }

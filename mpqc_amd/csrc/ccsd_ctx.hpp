@@ -279,6 +279,12 @@ class CCSDContext {
   bool pp_checked_ = false, pp_sym_ok_ = false;  // Gabcd's pair symmetry checked / holds
   bool pp_sym_planes_ = false;                   // the split forms' planes are the packed ones
   bool pp_symmetric_usable();
+  // o^2 v^4 from which the ladder runs on pairs where its alternative is one contraction: at
+  // o = 5, v = 32 (2.6e7) the packs and the unpack cost as much as the halved contraction saves,
+  // from 3e8 it is the faster by a fifth and more
+  static constexpr double kPairWork = 3.0e8;
+  bool tape_pairs();
+  void pp_ladder_transposed(const double* rbar, double* out, bool add, GemmPrecision prec);
   int2 *pv_sym_ = nullptr, *pv_anti_ = nullptr, *po_sym_ = nullptr, *po_anti_ = nullptr;
   double *Gpk_ = nullptr, *Gmk_ = nullptr, *WPk_ = nullptr, *WMk_ = nullptr;  // W_oooo's G+/- and products
   Planes Gp_P_sym_, Gm_P_sym_;

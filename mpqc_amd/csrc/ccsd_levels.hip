@@ -34,7 +34,6 @@ constexpr double kLvWideWork = 3.0e7;  // multiply-adds from which an op gets 64
 // multiply-adds, or if its tiles alone fill the chip:
 constexpr double kLvOwnWork = 2.0e8;
 constexpr long kLvOwnGroups = 300;
-constexpr double kLvPairWork = 3.0e8;  // from here the particle-particle ladder runs on symmetric pairs
 
 }  // namespace
 
@@ -207,7 +206,7 @@ void CCSDContext::plan_levels() {
   tape_execute_ = true;
   tau_fresh_ = fresh;
 
-  const bool psym = (double)v_ * v_ * v_ * v_ * o_ * o_ >= kLvPairWork && pp_symmetric_usable();
+  const bool psym = (double)v_ * v_ * v_ * v_ * o_ * o_ >= kPairWork && pp_symmetric_usable();
   if (psym && !pp_packed_) pack_pp_symmetric();
 
   // ---- ops with the buffers they read and write (buffers: allocation numbers; partial

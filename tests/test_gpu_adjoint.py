@@ -203,3 +203,26 @@ def test_products_repeat_bitwise(no, nv):
         assert np.array_equal(p[0], q[0]) and np.array_equal(p[1], q[1])
     for name in grad:
         assert np.array_equal(grad[name], grad2[name]), name
+
+
+# the ladder of the recorded residual and of the sweep on symmetric pairs (o^2 v^4 >= 3e8)
+# against the full contractions; without the pair symmetry both run in full
+@pytest.mark.parametrize("no,nv,symmetric", [(9, 45, True), (6, 61, True), (9, 45, False)])
+def test_products_on_pairs_match_full_ladder(no, nv, symmetric):
+    from mpqc_amd.ccsd import CCSD, Integrals
+    f, b = _random_case(no, nv, seed=no + nv)
+    rng = np.random.default_rng(no * nv)
+    if not symmetric:
+        b["Gabcd"] = b["Gabcd"] + rng.normal(0, 0.01, b["Gabcd"].shape)
+    t1, t2 = rng.normal(0, 0.02, (nv, no)), rng.normal(0, 0.02, (nv, nv, no, no))
+    y1, y2 = rng.normal(0, 1, (nv, no)), rng.normal(0, 1, (nv, nv, no, no))
+    got = {}
+    for pairs in (1, 0):
+        with CCSD(no, nv) as c:
+            c.set_integrals(Integrals(**b))
+            c.set_option("pp_symmetric", pairs)
+            c.set_amplitudes(t1, t2)
+            got[pairs] = c.jacobian_transpose(y1, y2) + c.get_residuals()
+    # FP64 sums of at most 2 v^2 products in another order
+    for x, y in zip(got[1], got[0]):
+        assert np.abs(x - y).max() <= 1e-12 * max(np.abs(y).max(), 1.0)

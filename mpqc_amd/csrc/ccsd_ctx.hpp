@@ -84,6 +84,8 @@ class CCSDContext {
   // ccsd_t.h:144-176, "straight" algorithm :1127-1167); seconds (optional) gets the
   // device time
   double triples(double block_bytes, double* seconds);
+  std::vector<double> triples_summed(double block_bytes);
+  std::vector<double> triples_orderings(double block_bytes);
   double triples_block_bytes_ = 8.0 * (1 << 30);
   // EOM-EE-CCSD singlet excitation energies (EOM_CCSD, eom_ccsd.h:17 with
   // eom_ccsd_impl.h:236-390): the lowest n_roots eigenvalues of the CCSD

@@ -110,3 +110,62 @@ def test_triples_split_precision_forms(prec, tol):
         esp, _ = c.triples()
     print(f"{prec} water: {esp:.12e} f64 {e64:.12e} diff {esp - e64:.2e}")
     assert abs(esp - e64) < tol * abs(e64)
+
+
+# tiles of the summed t3s: one column block, v on either side of a block's edge, wide tiles,
+# two tiles of columns (v > 144), K = v + o short of, at and past a multiple of 16; blocks of a few
+# triples with a shorter last one
+@pytest.mark.parametrize("no,nv,block_bytes", [(3, 13, 0), (4, 16, 1 << 20), (3, 17, 0), (5, 31, 1 << 20), (2, 81, 0),
+                                               (2, 145, 0)])
+def test_triples_sums_at_tile_edges(no, nv, block_bytes):
+    from mpqc_amd.ccsd import CCSD
+    rng = np.random.default_rng(no + nv)
+    naux = 6  # density-fitted blocks: <ia|bc> is built on the device, and no v^4 block is needed
+    X = rng.normal(0, 0.1, (naux, no + nv, no + nv))
+    X = 0.5 * (X + X.transpose(0, 2, 1))
+    o, v = slice(0, no), slice(no, no + nv)
+    eri = lambda p, q, r, s: np.einsum("Kpr,Kqs->pqrs", X[:, p, r], X[:, q, s])  # noqa: E731  <pq|rs>
+    eo, ev = np.sort(rng.uniform(-1.5, -0.4, no)), np.sort(rng.uniform(0.3, 2.5, nv))
+    b = {"Fia": np.zeros((no, nv)), "Fij": np.diag(eo), "Fab": np.diag(ev), "Gijab": eri(o, o, v, v),
+         "Gijkl": eri(o, o, o, o), "Giajb": eri(o, v, o, v), "Gijka": eri(o, o, o, v),
+         "Xai": X[:, v, o], "Xij": X[:, o, o], "Xab": X[:, v, v]}
+    t1, t2 = rng.normal(0, 0.05, (nv, no)), rng.normal(0, 0.05, (nv, nv, no, no))
+    ref = T.ccsd_t_straight(t1, t2, b["Gijab"], eri(o, v, v, v), b["Gijka"], eo, ev)
+    with CCSD(no, nv) as c:
+        c.set_df_basis(naux)
+        c.set_integrals({k: np.ascontiguousarray(x) for k, x in b.items()})
+        c.set_orbital_energies(eo, ev)
+        if block_bytes:
+            c.set_option("triples_block_bytes", block_bytes)
+        c.set_amplitudes(t1, t2)
+        et, _ = c.triples()
+        again, _ = c.triples()
+    assert et == again
+    assert abs(et - ref) < 1e-12 * abs(ref)
+
+
+# W of every ordering from 16-bit planes (v + o above the limit up to which the FP64 sums are the
+# faster, K not a multiple of 8) against the FP64 sums
+@pytest.mark.parametrize("prec,tol", [("f16x3", 5e-8), ("bf16x3", 1e-6)])  # as the split forms' test above
+def test_triples_from_planes_of_a_large_k(prec, tol):
+    from mpqc_amd.ccsd import CCSD
+    no, nv, naux = 2, 161, 6
+    rng = np.random.default_rng(no + nv)
+    X = rng.normal(0, 0.1, (naux, no + nv, no + nv))
+    X = 0.5 * (X + X.transpose(0, 2, 1))
+    o, v = slice(0, no), slice(no, no + nv)
+    eri = lambda p, q, r, s: np.einsum("Kpr,Kqs->pqrs", X[:, p, r], X[:, q, s])  # noqa: E731  <pq|rs>
+    eo, ev = np.sort(rng.uniform(-1.5, -0.4, no)), np.sort(rng.uniform(0.3, 2.5, nv))
+    b = {"Fia": np.zeros((no, nv)), "Fij": np.diag(eo), "Fab": np.diag(ev), "Gijab": eri(o, o, v, v),
+         "Gijkl": eri(o, o, o, o), "Giajb": eri(o, v, o, v), "Gijka": eri(o, o, o, v),
+         "Xai": X[:, v, o], "Xij": X[:, o, o], "Xab": X[:, v, v]}
+    t1, t2 = rng.normal(0, 0.05, (nv, no)), rng.normal(0, 0.05, (nv, nv, no, no))
+    et = {}
+    for p in ("f64", prec):
+        with CCSD(no, nv, precision=p) as c:
+            c.set_df_basis(naux)
+            c.set_integrals({k: np.ascontiguousarray(x) for k, x in b.items()})
+            c.set_orbital_energies(eo, ev)
+            c.set_amplitudes(t1, t2)
+            et[p], _ = c.triples()
+    assert 0 < abs(et[prec] - et["f64"]) < tol * abs(et["f64"])

@@ -143,17 +143,41 @@ __global__ __launch_bounds__(kSymBlock) void unpack_ladder_kernel(double* __rest
 }
 
 // per block, over G with extents (p, p, q, q): max |G(a,b,c,d) - G(b,a,d,c)| and
-// max |G(a,b,c,d)| -> part[2 blk], part[2 blk + 1]
+// max |G(a,b,c,d)| -> part[2 blk], part[2 blk + 1].  A 32 x 32 tile of (c,d) of row a <= b against
+// the transposed tile of row (b,a), through LDS: every element is read once, in whole lines.
+// Bound: HBM (16 hydrogen chains, 5.3 GB: 7.0 ms element by element, each with its partner and
+// six divisions, 1.5 ms so).  NaN: fmax drops it, but a NaN integral has made the result NaN
+// either way.
+constexpr int kSymTile = 32;
 __global__ __launch_bounds__(kSymBlock) void pair_asymmetry_kernel(double* __restrict__ part,
-                                                                   const double* __restrict__ G, long p, long q) {
+                                                                   const double* __restrict__ G, int p, int q) {
+  __shared__ double tile[kSymTile][kSymTile + 1];
   __shared__ double sd[kSymBlock], sg[kSymBlock];
-  const long total = p * p * q * q;
+  const int tiles = (q + kSymTile - 1) / kSymTile, x = threadIdx.x % kSymTile, y0 = threadIdx.x / kSymTile;
+  const long qq = (long)q * q, items = (long)p * p * tiles * tiles;
   double md = 0.0, mg = 0.0;
-  for (long e = (long)blockIdx.x * kSymBlock + threadIdx.x; e < total; e += (long)gridDim.x * kSymBlock) {
-    const long d = e % q, t0 = e / q, c = t0 % q, t1 = t0 / q, b = t1 % p, a = t1 / p;
-    const double x = G[e];
-    md = fmax(md, fabs(x - G[((b * p + a) * q + d) * q + c]));
-    mg = fmax(mg, fabs(x));
+  for (long it = blockIdx.x; it < items; it += gridDim.x) {
+    const long ab = it / (tiles * tiles);
+    const int t = (int)(it - ab * tiles * tiles), a = (int)(ab / p), b = (int)(ab - (long)a * p);
+    if (a > b) continue;
+    const int c0 = t / tiles * kSymTile, d0 = t % tiles * kSymTile;
+    const double* const g1 = G + ab * qq;
+    const double* const g2 = G + ((long)b * p + a) * qq;
+    double g[kSymTile * kSymTile / kSymBlock];
+#pragma unroll
+    for (int k = 0; k < kSymTile * kSymTile / kSymBlock; ++k) {
+      const int y = y0 + k * (kSymBlock / kSymTile);
+      g[k] = c0 + y < q && d0 + x < q ? g1[(long)(c0 + y) * q + d0 + x] : 0.0;
+      tile[y][x] = d0 + y < q && c0 + x < q ? g2[(long)(d0 + y) * q + c0 + x] : 0.0;
+    }
+    __syncthreads();
+#pragma unroll
+    for (int k = 0; k < kSymTile * kSymTile / kSymBlock; ++k) {
+      const double h = tile[x][y0 + k * (kSymBlock / kSymTile)];
+      md = fmax(md, fabs(g[k] - h));
+      mg = fmax(mg, fmax(fabs(g[k]), fabs(h)));
+    }
+    __syncthreads();
   }
   sd[threadIdx.x] = md;
   sg[threadIdx.x] = mg;
@@ -201,6 +225,9 @@ __global__ __launch_bounds__(kSymBlock) void swap13_asymmetry_kernel(double* __r
   }
 }
 
+constexpr long kCheckBlocks = 2048;  // workgroups of a symmetry check: fill the chip, 32 KB of maxima back
+static_assert(2 * kCheckBlocks <= kReducePartials, "partials");
+
 int sym_grid(long n) { return (int)std::max<long>(1, std::min<long>(ceil_div(n, kSymBlock), 65536)); }
 
 std::vector<int2> pair_table(long n, bool strict) {
@@ -222,8 +249,8 @@ bool CCSDContext::pp_symmetric_usable() {
   if (pp_checked_) return pp_sym_ok_;
   // whether G with extents (p, p, q, q) holds G(b,a,d,c) = G(a,b,c,d) to 1e-12 of its largest element
   auto symmetric = [&](const double* G, long p, long q) {
-    const int blocks = (int)std::max<long>(1, std::min<long>(ceil_div(p * p * q * q, kSymBlock), kReducePartials / 2));
-    hipLaunchKernelGGL(pair_asymmetry_kernel, dim3(blocks), dim3(kSymBlock), 0, stream_, partials_, G, p, q);
+    const int blocks = (int)std::max<long>(1, std::min<long>(p * p * ceil_div(q, kSymTile) * ceil_div(q, kSymTile), kCheckBlocks));
+    hipLaunchKernelGGL(pair_asymmetry_kernel, dim3(blocks), dim3(kSymBlock), 0, stream_, partials_, G, (int)p, (int)q);
     check_launch("pair_asymmetry");
     std::vector<double> h(2 * (size_t)blocks);
     MPQC_HIP_CHECK(hipMemcpyAsync(h.data(), partials_, h.size() * sizeof(double), hipMemcpyDeviceToHost, stream_));
@@ -250,7 +277,7 @@ bool CCSDContext::pp_symmetric_usable() {
 bool CCSDContext::giabc_symmetric_usable() {
   if (iabc_checked_) return iabc_sym_ok_;
   const long total = (long)o_ * v_ * v_ * v_;
-  const int blocks = (int)std::max<long>(1, std::min<long>(ceil_div(total, kSymBlock), kReducePartials / 2));
+  const int blocks = (int)std::max<long>(1, std::min<long>(ceil_div(total, kSymBlock), kCheckBlocks));
   hipLaunchKernelGGL(swap13_asymmetry_kernel, dim3(blocks), dim3(kSymBlock), 0, stream_, partials_, Giabc_,
                      (long)o_, (long)v_, (long)v_);
   check_launch("swap13_asymmetry");
@@ -277,27 +304,46 @@ void CCSDContext::pack_pp_symmetric() {
   ldvs_ = pad64(nvs_);
   ldva_ = pad64(nva_);
   if (!pv_sym_) {
-    auto upload_pairs = [&](long n, bool strict) {
-      const std::vector<int2> t = pair_table(n, strict);
-      int2* d = reinterpret_cast<int2*>(alloc(std::max<size_t>(t.size(), 1)));
-      if (!t.empty())
-        MPQC_HIP_CHECK(hipMemcpyAsync(d, t.data(), t.size() * sizeof(int2), hipMemcpyHostToDevice, stream_));
-      return d;
-    };
-    pv_sym_ = upload_pairs(V, false);
-    pv_anti_ = upload_pairs(V, true);
-    po_sym_ = upload_pairs(O, false);
-    po_anti_ = upload_pairs(O, true);
-    Vpk_ = alloc((size_t)nvs_ * ldvs_);
-    Vmk_ = alloc((size_t)std::max<long>(nva_, 1) * ldva_);
-    Spk_ = alloc((size_t)oo * ldvs_);
-    Apk_ = alloc((size_t)oo * ldva_);
-    Ppk_ = alloc((size_t)nvs_ * oo);
-    Mpk_ = alloc((size_t)std::max<long>(nva_, 1) * oo);
-    Gpk_ = alloc((size_t)nos_ * ldvs_);
-    Gmk_ = alloc((size_t)std::max<long>(noa_, 1) * ldva_);
-    WPk_ = alloc((size_t)nos_ * oo);
-    WMk_ = alloc((size_t)std::max<long>(noa_, 1) * oo);
+    // one allocation and one upload (a first pass that makes 14 of them spends its time there:
+    // 16 hydrogen chains side by side: 2.4 ms of a first pass of 25.6)
+    std::vector<int2> table;
+    size_t at[4];
+    int k = 0;
+    for (long n : {V, O})
+      for (bool strict : {false, true}) {
+        const std::vector<int2> t = pair_table(n, strict);
+        at[k++] = table.size();
+        table.insert(table.end(), t.begin(), t.end());
+      }
+    const size_t n2 = table.size(), va = std::max<long>(nva_, 1), oa = std::max<long>(noa_, 1);
+    const size_t sizes[11] = {n2,          (size_t)(nvs_ * ldvs_), va * ldva_,         (size_t)(oo * ldvs_),
+                              (size_t)(oo * ldva_), (size_t)(nvs_ * oo),    va * oo,  (size_t)(nos_ * ldvs_),
+                              oa * ldva_,  (size_t)(nos_ * oo),    oa * oo};
+    size_t total = 0;
+    for (size_t n : sizes) total += (n + 31) / 32 * 32;
+    double* p = alloc(total);
+    double* part[11];
+    for (int q = 0; q < 11; ++q) {
+      part[q] = p;
+      p += (sizes[q] + 31) / 32 * 32;
+    }
+    int2* d = reinterpret_cast<int2*>(part[0]);
+    MPQC_HIP_CHECK(hipMemcpyAsync(d, table.data(), n2 * sizeof(int2), hipMemcpyHostToDevice, stream_));
+    MPQC_HIP_CHECK(hipStreamSynchronize(stream_));  // (the table is this scope's)
+    Vpk_ = part[1];
+    Vmk_ = part[2];
+    Spk_ = part[3];
+    Apk_ = part[4];
+    Ppk_ = part[5];
+    Mpk_ = part[6];
+    Gpk_ = part[7];
+    Gmk_ = part[8];
+    WPk_ = part[9];
+    WMk_ = part[10];
+    pv_anti_ = d + at[1];
+    po_sym_ = d + at[2];
+    po_anti_ = d + at[3];
+    pv_sym_ = d + at[0];
   }
   hipLaunchKernelGGL(pack_pairs_kernel, dim3(sym_grid(nvs_ * ldvs_)), dim3(kSymBlock), 0, stream_, Vpk_, Gabcd_, V, V,
                      pv_sym_, nvs_, pv_sym_, nvs_, ldvs_, 1.0);

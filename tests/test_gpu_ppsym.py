@@ -90,3 +90,26 @@ def test_asymmetric_blocks_take_the_full_contraction(prec, bar, block):
     e2 = np.abs(r2 - r2r).max() / np.abs(r2r).max()
     print(f"asymmetric {block} {prec}: r1 {e1:.2e} r2 {e2:.2e}")
     assert e1 < bar and e2 < bar
+
+
+# one element off its partner, inside a tile of the check, at its edge and in the last, partial one:
+# found wherever it is (the full contraction then runs and matches the oracle)
+@pytest.mark.parametrize("index", [(0, 1, 2, 3), (3, 2, 31, 32), (5, 5, 0, 36), (36, 36, 36, 35), (36, 0, 32, 36)])
+def test_symmetry_check_finds_a_single_element(index):
+    from mpqc_amd.ccsd import CCSD, Integrals
+    from spinorb_ccsd import mpqc_blocks, random_hamiltonian
+    no, nv = 2, 37
+    f, g = random_hamiltonian(no, nv, seed=5, eri_scale=0.03)
+    b = mpqc_blocks(f, g, no)
+    b["Gabcd"] = b["Gabcd"].copy()
+    b["Gabcd"][index] += 0.5
+    rng = np.random.default_rng(6)
+    t1, t2 = rng.normal(0, 0.02, (nv, no)), rng.normal(0, 0.02, (nv, nv, no, no))
+    got = []
+    for pairs in (1, 0):
+        with CCSD(no, nv) as c:
+            c.set_option("levels", 0)
+            c.set_option("pp_symmetric", pairs)
+            c.set_integrals(Integrals(**b))
+            got.append(c.compute_residuals(t1, t2))
+    assert np.array_equal(got[0][1], got[1][1])  # both ran the full contraction

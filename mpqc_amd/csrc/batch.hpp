@@ -6,7 +6,9 @@
 // sizes), so op k of all molecules becomes one grouped launch: a persistent
 // grouped contraction over every molecule's output tiles, or one grouped
 // permutation / copy / tau build.  The launch sequence is captured in a
-// hipGraph once and replayed for every batched residual.  Each grouped
+// hipGraph once and replayed for every batched residual.  Batches of few or large
+// molecules run the molecules' own residuals on their own streams instead
+// (side_by_side()).  Each grouped
 // contraction's tile edge and split-K target are chosen by an autotuner that
 // times the candidates on the batch itself.
 #pragma once
@@ -72,6 +74,10 @@ class CCSDBatch {
   GemmPrecision prec_ = GemmPrecision::F64;
 
   void plan();
+  bool side_by_side();
+  void launch_side_by_side();
+  void sync_molecules();
+  int side_ = -1;  // whether the molecules run side by side (-1: not chosen yet)
   void ensure_planned();
   void build_plan(Stage& s);
   void launch_stage(const Stage& s);

@@ -93,3 +93,25 @@ def test_batched_hchains_match_single_molecule_path():
             assert _rel(r1, o1) < 1e-12 and _rel(r2, o2) < 1e-12
         st = B.stages()
         assert sum(s["kind"] == "contraction" for s in st) > 30
+
+
+# many small molecules in grouped launches; few, among them one whose ladder runs on pairs, side by
+# side; either way over repeated passes, new amplitudes and new integrals of one molecule
+@pytest.mark.parametrize("sizes", [[(2, 7), (1, 5), (3, 6)] * 8, [(9, 45), (2, 7), (5, 13)]])
+def test_grouped_and_side_by_side_match_oracle(sizes):
+    from mpqc_amd.batch import CCSDBatch
+    mols, rng = _random_batch(sizes, seed=70)
+    with CCSDBatch([s[0] for s in sizes], [s[1] for s in sizes]) as B:
+        for k, b in enumerate(mols):
+            B.set_integrals(k, b)
+        for rnd in range(4):
+            if rnd == 3:
+                mols[1] = _random_batch([sizes[1]], seed=99)[0][0]
+                B.set_integrals(1, mols[1])
+            amps = [_amplitudes(rng, no, nv) for no, nv in sizes]
+            for k, (t1, t2) in enumerate(amps):
+                B.set_amplitudes(k, t1, t2)
+            B.residual()
+            for k, (t1, t2) in enumerate(amps):
+                got, ref = B.get_residuals(k), _oracle_residual(mols[k], t1, t2)
+                assert _rel(got[0], ref[0]) < 1e-12 and _rel(got[1], ref[1]) < 1e-12, (rnd, k)

@@ -184,7 +184,6 @@ void CCSDContext::construct(const int64_t* occ_hm, int n_occ_tiles, const int64_
   partials_ = alloc(kReducePartials);
   scalars_ = alloc(64);
   MPQC_HIP_CHECK(hipGetDevice(&device_));
-  MPQC_HIP_CHECK(hipHostMalloc((void**)&host_scalars_, 64 * sizeof(double), hipHostMallocDefault));
   if (with_solver) solver_init(1, 8, 0.0, 1, 1);
   MPQC_HIP_CHECK(hipMemsetAsync(t1_, 0, ov * sizeof(double), stream_));
   MPQC_HIP_CHECK(hipMemsetAsync(t2_, 0, oovv * sizeof(double), stream_));
@@ -1464,8 +1463,15 @@ std::vector<int> CCSDContext::diis_kept(int* slot) const {
   return kept;
 }
 
+// (allocated at first use: molecules of a batch and operator-interface contexts never need it)
+double* CCSDContext::host_scalars() {
+  if (!host_scalars_) MPQC_HIP_CHECK(hipHostMalloc((void**)&host_scalars_, 64 * sizeof(double), hipHostMallocDefault));
+  return host_scalars_;
+}
+
 void CCSDContext::energy_error(double* E, double* err, std::vector<double>* dots) {
   if (!prepared_) prepare();
+  double* const h = host_scalars();
   const long n1 = (long)o_ * v_, n2 = n1 * n1;
   // error = sqrt(|r1|^2 + |r2|^2) / (size(r1) + size(r2))   qc/cc/solvers.h:60-63
   // E = 2 <f_ai + r1, t1> + <g_abij + r2, 2 tau(a,b,i,j) - tau(b,a,i,j)>   ccsd.h:377-379
@@ -1484,15 +1490,14 @@ void CCSDContext::energy_error(double* E, double* err, std::vector<double>* dots
     }
     timed("en:energy_dots", 0.0, [&] {
       ccsd_energy_dots(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, x1.data(), x2.data(), nvec, hist_e1_[slot],
-                       hist_e2_[slot], host_scalars_, partials_, stream_);
+                       hist_e2_[slot], h, partials_, stream_);
     });
   } else {
     timed("en:energy", 0.0, [&] {
-      ccsd_energy_norms(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, host_scalars_, partials_, stream_);
+      ccsd_energy_norms(f_ai_, r1_, t1_, g_abij_, r2_, tau_, o_, v_, h, partials_, stream_);
     });
   }
   MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
-  const double* h = host_scalars_;
   const double e = std::sqrt(h[0] + h[1]) / (double)(n1 + n2);
   if (!std::isfinite(e) || !std::isfinite(h[2]))
     throw std::range_error("non-finite residual or energy");
@@ -1533,11 +1538,13 @@ void CCSDContext::update(const std::vector<double>* dots) {
   err_slots_.push_back(eslot);
   const int nvec = (int)err_slots_.size();
   {
-    const double* h = host_scalars_ + 32;
+    const double* h = nullptr;
     if (dots) {
       if ((int)dots->size() != nvec) throw std::logic_error("DIIS: overlaps of another history");
       h = dots->data();
     } else {
+      double* const sums = host_scalars() + 32;
+      h = sums;
       // the new error vector r goes into its slot in the pass that forms its overlaps with
       // the history (its own overlap read from r itself)
       std::vector<const double*> x1, x2;
@@ -1546,7 +1553,7 @@ void CCSDContext::update(const std::vector<double>* dots) {
         x2.push_back(s == eslot ? r2_ : hist_e2_[s]);
       }
       timed("up:diis_dots", 0.0, [&] {
-        multi_dot2(x1.data(), x2.data(), nvec, r1_, r2_, n1, n2, host_scalars_ + 32, partials_, stream_, hist_e1_[eslot],
+        multi_dot2(x1.data(), x2.data(), nvec, r1_, r2_, n1, n2, sums, partials_, stream_, hist_e1_[eslot],
                    hist_e2_[eslot]);
       });
       MPQC_HIP_CHECK(hipStreamSynchronize(stream_));

@@ -352,6 +352,7 @@ class CCSDContext {
   double* scalars_ = nullptr;  // device scalars
   // pinned host memory that the last pass of a reduction writes (no copy back to wait for)
   double* host_scalars_ = nullptr;
+  double* host_scalars();
   // DIIS error vectors that stay when one is pushed, and the slot the new one takes
   std::vector<int> diis_kept(int* slot) const;
   long* modeinfo_ = nullptr;   // device tile maps (scratch, sized per call)

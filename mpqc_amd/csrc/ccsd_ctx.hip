@@ -1212,7 +1212,9 @@ void CCSDContext::residual_ops() {
   // also stands for Rd's term (a T1 dressing term in 16-bit planes slows the split forms'
   // convergence: (H2O)8 bf16x3 36 iterations to 1e-8 instead of 18)
   auto j_giabc_t1 = [&] {
-    if (sm && !iabc_sym && !Giabc_P_.row)  // (padded rows hold (c,d) pairs, not d alone)
+    // (planes only where neither operand is padded: Giabc's padded rows hold (c,d) pairs, t1's d
+    // alone, and v = 4 (mod 8) pads only the latter)
+    if (sm && !iabc_sym && !Giabc_P_.row && !t1T_P_.row)
       gemmP(o * v * v, o, v, 1.0, Giabc_P_, v, t1T_P_, v, 0.0, Zj_, o, "r2:j_giabc_t1");
     else
       gemm(false, false, o * v * v, o, v, 1.0, Giabc_, v, t1_, o, 0.0, Zj_, o, 0, 0, 0, 1, "r2:j_giabc_t1");

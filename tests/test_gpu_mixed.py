@@ -133,12 +133,14 @@ def test_deep_pipeline_plane_kernel_residual(prec):
 
 
 @pytest.mark.parametrize("prec", ["f16x3", "bf16x3", "bf16x6"])
-@pytest.mark.parametrize("no,nv,symmetric", [(7, 37, True), (5, 53, True), (6, 44, True), (8, 33, False), (1, 9, True)])
+@pytest.mark.parametrize("no,nv,symmetric", [(7, 37, True), (5, 53, True), (6, 44, True), (8, 33, False), (1, 9, True),
+                                             (6, 44, False), (3, 12, False), (8, 20, False), (5, 42, False), (8, 40, False)])
 def test_padded_plane_rows_residual(prec, no, nv, symmetric):
     """Orbital counts whose o^2, v^2, o v or v is no multiple of 8, so the planes' rows are
     padded: odd ones, an even v with o v a multiple of 8, one occupied orbital, and
-    integrals without Giabc(i,c,a,b) = Giabc(i,b,a,c) (its T1 term then leaves the planes);
-    against the oracle within the form's bound."""
+    integrals without Giabc(i,c,a,b) = Giabc(i,b,a,c) at every way in which v and v^2 can be
+    padded (v odd; 2, 4 or 0 mod 8: v^2 padded, v alone, neither); against the oracle within
+    the form's bound."""
     from oracle import ccsd as O
     from mpqc_amd.ccsd import CCSD, Integrals
     from spinorb_ccsd import mpqc_blocks, random_hamiltonian

@@ -629,16 +629,22 @@ std::vector<double> CCSDContext::triples_summed(double block_bytes) {
   const long O = o_, V = v_, v3 = V * V * V, VK = V + O, pitch = ceil_div(VK, 16) * 16;
   const long ncube = energy_cubes(V), total = O * (O + 1) * (O + 2) / 6;
   // triples a block: as many t3s as fit (at most the memory of one (j,k)'s six orderings, beyond
-  // which the launches are long enough), in blocks of equal size within the energy's 2^31 workgroups
+  // which the launches are long enough), in blocks of equal size within the energy's 2^24 workgroups
+  // (2^32 threads of a launch)
   long T = std::max(1L, std::min({(long)(block_bytes / (sizeof(double) * (double)v3)), 6 * O, total,
-                                  ((1L << 31) - 1) / ncube - 8}));
+                                  (1L << 24) / ncube - 8}));
   const long nchunks = ceil_div(total, T);
   T = ceil_div(total, nchunks);
   const size_t d = sizeof(double);
   ScratchBuf A(scratch_, (size_t)(O * V * V * pitch)), As(scratch_, (size_t)(O * V * V * pitch)),
       B(scratch_, (size_t)(O * O * V * pitch)), W(scratch_, (size_t)(T * v3));
   {
-    ScratchBuf tmp(scratch_, (size_t)std::max(O * V * V * std::max(V, O), O * O * V * std::max(V, O)));
+    // The operands' parts go through a temporary a few occupied orbitals at a time: with one for
+    // all of o v^3, the two A's would take more memory than one A and the W of every ordering,
+    // and fewer orbitals would fit the device.  128 MiB of it cost no time (at o = 20, v = 76 it holds
+    // all orbitals).
+    const long per = V * std::max(V, O) * std::max(V, O), step = std::max(1L, std::min(O, (16L << 20) / per));
+    ScratchBuf tmp(scratch_, (size_t)(step * per));
     if (pitch != VK) {
       fill(A.p, O * V * V * pitch, 0.0, stream_);
       fill(B.p, O * O * V * pitch, 0.0, stream_);
@@ -646,23 +652,28 @@ std::vector<double> CCSDContext::triples_summed(double block_bytes) {
     auto rows = [&](double* dst, long n, long width) {  // dst rows of `pitch` take tmp's rows of `width`
       MPQC_HIP_CHECK(hipMemcpy2DAsync(dst, pitch * d, tmp.p, width * d, width * d, n, hipMemcpyDeviceToDevice, stream_));
     };
-    // A[i][(a,b)][d] = Giabc(i,d,a,b), [v + l] = t2(a,b,i,l)
-    const long e_iabc[4] = {O, V, V, V}, e_t2[4] = {V, V, O, O}, e_a2[4] = {O, V, V, O};
-    const int pa1[4] = {0, 2, 3, 1}, pa2[4] = {2, 0, 1, 3};
-    permute_into(tmp.p, e_iabc, Giabc_, e_iabc, pa1, 1.0, stream_);
-    rows(A.p, O * V * V, V);
-    permute_into(tmp.p, e_a2, t2_, e_t2, pa2, 1.0, stream_);
-    rows(A.p + V, O * V * V, O);
+    const long e_iabc[4] = {O, V, V, V}, e_t2[4] = {V, V, O, O}, e_ijka[4] = {O, O, O, V};
+    const int pa1[4] = {0, 2, 3, 1}, pa2[4] = {2, 0, 1, 3}, pb1[4] = {2, 3, 1, 0}, pb2[4] = {0, 1, 3, 2};
+    for (long i0 = 0; i0 < O; i0 += step) {
+      const long n = std::min(step, O - i0);
+      // A[i][(a,b)][d] = Giabc(i,d,a,b), [v + l] = t2(a,b,i,l)
+      const long e_a1[4] = {n, V, V, V}, e_a2[4] = {n, V, V, O};
+      double* const a = A.p + i0 * V * V * pitch;
+      permute_into(tmp.p, e_a1, Giabc_ + i0 * v3, e_iabc, pa1, 1.0, stream_);
+      rows(a, n * V * V, V);
+      permute_into(tmp.p, e_a2, t2_ + i0 * O, e_t2, pa2, 1.0, stream_);
+      rows(a + V, n * V * V, O);
+      // B[j][k][c][d] = t2(d,c,j,k), [v + l] = -Gijka(j,k,l,c)
+      const long e_b1[4] = {n, O, V, V}, e_b2[4] = {n, O, V, O};
+      double* const b = B.p + i0 * O * V * pitch;
+      permute_into(tmp.p, e_b1, t2_ + i0 * O, e_t2, pb1, 1.0, stream_);
+      rows(b, n * O * V, V);
+      permute_into(tmp.p, e_b2, Gijka_ + i0 * O * O * V, e_ijka, pb2, -1.0, stream_);
+      rows(b + V, n * O * V, O);
+    }
     const long e_a[4] = {O, V, V, pitch};
     const int psw[4] = {0, 2, 1, 3};
     permute_into(As.p, e_a, A.p, e_a, psw, 1.0, stream_);
-    // B[j][k][c][d] = t2(d,c,j,k), [v + l] = -Gijka(j,k,l,c)
-    const long e_b1[4] = {O, O, V, V}, e_ijka[4] = {O, O, O, V}, e_b2[4] = {O, O, V, O};
-    const int pb1[4] = {2, 3, 1, 0}, pb2[4] = {0, 1, 3, 2};
-    permute_into(tmp.p, e_b1, t2_, e_t2, pb1, 1.0, stream_);
-    rows(B.p, O * O * V, V);
-    permute_into(tmp.p, e_b2, Gijka_, e_ijka, pb2, -1.0, stream_);
-    rows(B.p + V, O * O * V, O);
   }
   // tables of the cube and triple multisets
   const long nB = ceil_div(V, kT);

@@ -169,3 +169,52 @@ def test_triples_from_planes_of_a_large_k(prec, tol):
             c.set_amplitudes(t1, t2)
             et[p], _ = c.triples()
     assert 0 < abs(et[prec] - et["f64"]) < tol * abs(et["f64"])
+
+
+def test_triples_operands_in_parts():
+    """Operands that are set up a few occupied orbitals at a time (o max(v, o)^2 v > 2^24): the energy
+    against that from fp16 planes, and no more device memory than one A with K = v + o, its
+    o v^3 temporary, six B, the six orderings of W for one i and a permuted Gijka."""
+    import ctypes
+    import torch
+    from mpqc_amd import _lib as L
+    from mpqc_amd.ccsd import CCSD
+    no, nv, naux = 12, 160, 6
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    new = lambda *s: torch.randn(s, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    X = 0.05 * new(naux, no + nv, no + nv)
+    X = X + X.transpose(1, 2)
+    o, v = slice(0, no), slice(no, no + nv)
+
+    def eri(p, q, r, s):  # <pq|rs>
+        A, B = X[:, p, r], X[:, q, s]
+        g = A.reshape(naux, -1).T @ B.reshape(naux, -1)
+        return g.reshape(A.shape[1], A.shape[2], B.shape[1], B.shape[2]).permute(0, 2, 1, 3).contiguous()
+
+    rng = np.random.default_rng(4)
+    eo, ev = np.sort(rng.uniform(-1.5, -0.4, no)), np.sort(rng.uniform(0.3, 2.5, nv))
+    dev = lambda x: torch.from_numpy(x).cuda()  # noqa: E731
+    blocks = {"Fia": dev(np.zeros((no, nv))), "Fij": dev(np.diag(eo)), "Fab": dev(np.diag(ev)),
+              "Gijab": eri(o, o, v, v), "Gijkl": eri(o, o, o, o), "Giajb": eri(o, v, o, v),
+              "Giabc": eri(o, v, v, v), "Gijka": eri(o, o, o, v), "Gabcd": eri(v, v, v, v)}
+    t1, t2 = 0.05 * new(nv, no), 0.05 * new(nv, nv, no, no)
+    torch.cuda.synchronize()
+    p = lambda t: ctypes.c_void_p(t.data_ptr())  # noqa: E731
+    et = {}
+    for prec in ("f64", "f16x3"):
+        with CCSD(no, nv, precision=prec) as c:
+            for name, t in blocks.items():
+                c._check(c.lib.mpqc_ccsd_set_integral(c.ctx, L.INTEGRAL_IDS[name], p(t), L.LAYOUT_DENSE, L.MEM_DEVICE))
+            c.set_orbital_energies(eo, ev)
+            c.set_option("triples_block_bytes", 1 << 20)
+            c.init_guess()  # derived integral layouts exist
+            c._check(c.lib.mpqc_ccsd_set_amplitudes(c.ctx, p(t1), p(t2), L.LAYOUT_DENSE, L.MEM_DEVICE))
+            before = torch.cuda.mem_get_info()[0]
+            et[prec], _ = c.triples()
+            if prec == "f64":  # (the context keeps up to 4 GiB of temporaries)
+                used = before - torch.cuda.mem_get_info()[0]
+                k, v3 = nv + no, nv ** 3
+                most = no * nv * nv * k + no * v3 + 6 * no * no * nv * k + 6 * v3 + no * no * nv * nv
+                print(f"scratch {used / 2**20:.0f} MiB of {most * 8 / 2**20:.0f}")
+                assert used <= 8 * most
+    assert 0 < abs(et["f16x3"] - et["f64"]) < 5e-8 * abs(et["f64"])  # as the split forms' test above

@@ -376,6 +376,7 @@ struct F64Plan {
 };
 
 constexpr int kCUs = 256;
+constexpr long kMaxThreads = 1L << 32;  // of a launch, per dimension
 
 F64Plan plan_f64(const GemmDesc& d, size_t ws_bytes) {
   const size_t slice_bytes = (size_t)d.M * d.N * sizeof(double);
@@ -385,7 +386,10 @@ F64Plan plan_f64(const GemmDesc& d, size_t ws_bytes) {
   for (int ti = 0; ti < kF64TileCount; ++ti) {
     const F64Tile& c = kF64Tiles[ti];
     const long slices = ceil_div(d.K, 16 * c.u);
-    const long work = ceil_div(d.M, 64 * c.rb) * ceil_div(d.N, 16 * c.cb) * d.batch;
+    const long tiles = ceil_div(d.M, 64 * c.rb) * ceil_div(d.N, 16 * c.cb), work = tiles * d.batch;
+    // (rows of A in the hundreds of millions: only the tiles whose grid, rounded up to the XCDs, can
+    // be launched; the first, largest one stands for a shape that none can take)
+    if (ti > 0 && (tiles + kXcdCount) * kThreads * c.kg >= kMaxThreads) continue;
     const double own = c.rb * c.cb * c.u * 256.0;  // products of a slice, per SIMD
     // splits that give each CU up to three workgroups, at least 128 values of k long
     long last = 0;

@@ -264,3 +264,22 @@ def test_gemm_f64_tiles(ta, tb, m, n, k, batch, beta):
     # each of k products and sums rounds once in either result: 2 k eps |A| |B|, and the scaling
     bound = 2 * (k + 4) * 2.3e-16 * (0.7 * (np.abs(a) @ np.abs(b)) + (abs(beta) * np.abs(C[:, :, :n]) if beta else 0.0))
     assert np.all(np.abs(got[:, :, :n] - ref[:, :, :n]) <= bound)
+
+
+def test_gemm_f64_rows_past_a_two_group_grid():
+    """So many rows that a grid of the narrow tiles with two K groups would pass the 2^32 threads of
+    a launch: a Toeplitz A (rows one element apart) against shifted sums."""
+    from mpqc_amd.ccsd import gemm
+    m, k = 540_000_000, 64
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    a = torch.randn(m + k, dtype=torch.float64, device="cuda", generator=gen)
+    b = torch.randn(k, dtype=torch.float64, device="cuda", generator=gen)
+    c = torch.empty(m, dtype=torch.float64, device="cuda")
+    torch.cuda.synchronize()
+    gemm(0, 1, m, 1, k, 1.0, a.data_ptr(), 1, b.data_ptr(), k, 0.0, c.data_ptr(), 1)
+    torch.cuda.synchronize()
+    for q, w in enumerate(b.cpu().tolist()):
+        c.add_(a[q:q + m], alpha=-w)
+    # each of k products and sums rounds once in either result
+    bound = 2 * (k + 4) * 2.3e-16 * float(a.abs().max()) * float(b.abs().sum())
+    assert float(c.abs().max()) <= bound

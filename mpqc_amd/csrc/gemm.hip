@@ -378,7 +378,45 @@ struct F64Plan {
 constexpr int kCUs = 256;
 constexpr long kMaxThreads = 1L << 32;  // of a launch, per dimension
 
+// A contraction with K <= 64 has at most four slices a tile: prologue and epilogue, which the model
+// below does not tell apart, are most of its time, and the smaller tiles are the better ones until
+// they take more rounds of the CUs.  It gets the tile with the least rounds * (blocks of 16 x 64
+// outputs + 2) of those that one K group works on with few registers (128 x 80 up to K = 48).  From
+// K = 33 outputs of up to 128 or more than 768 tiles of 64 x 64 stay with the model: K groups help the
+// former (2500 x 90 x 40: 5.1 us with two of them, 5.8 with 64 x 64 tiles), its wider tiles the latter
+// (3955 x 1417 x 52: 22.3 : 26.2).  Against the model's choice (us): 502 x 1490 x 15 6.1 -> 5.3, 2000 x
+// 2000 x 16 10.8 -> 10.2, 30000 x 361 x 19 30.6 -> 27.7, 3000 x 1000 x 36 13.3 -> 13.0, 20000 x 100 x 64 13.6 -> 12.3;
+// and 0.3 less host time for the smallest calls.
+constexpr int kShortK = 64;
+bool short_k_shape(const GemmDesc& d) {
+  const long tiles = ceil_div(d.M, 64) * ceil_div(d.N, 64) * d.batch;
+  return d.K <= 32 || (d.K <= kShortK && tiles > 128 && tiles <= 3 * kCUs);
+}
+
+int short_k_tile(const GemmDesc& d) {
+  int best = 0;
+  long best_cost = -1;
+  for (int ti = 0; ti < kF64TileCount; ++ti) {
+    const F64Tile& c = kF64Tiles[ti];
+    const bool small = c.rb == 1 && c.kg == 1 && c.cb <= 8, wide = c.rb == 2 && c.cb == 5 && d.K <= 48;
+    if (!small && !wide) continue;
+    const long tiles = ceil_div(d.M, 64 * c.rb) * ceil_div(d.N, 16 * c.cb);
+    const long cost = ceil_div(tiles * d.batch, kCUs) * (c.rb * c.cb + 2);
+    if (best_cost < 0 || cost <= best_cost) {
+      best = ti;
+      best_cost = cost;
+    }
+  }
+  return best;
+}
+
 F64Plan plan_f64(const GemmDesc& d, size_t ws_bytes) {
+  if (short_k_shape(d)) {
+    F64Plan p;
+    p.tile = short_k_tile(d);
+    p.kchunk = (int)(ceil_div(d.K, 16 * kF64Tiles[p.tile].u) * 16 * kF64Tiles[p.tile].u);
+    return p;
+  }
   const size_t slice_bytes = (size_t)d.M * d.N * sizeof(double);
   const double hbm = ((double)d.M * d.K + (double)d.K * d.N + (double)d.M * d.N) * d.batch * 8.0 / 2100.0;
   F64Plan best;

@@ -236,12 +236,16 @@ def test_gemm_split_error_bound(prec, ta, tb, m, n, k):
 
 # FP64 tile kernel: one size per tile of the planner (64 or 128 rows, 16 to 144 columns, one
 # to four K groups), odd N (the last 16-byte piece of a row of B), N of 1, K that ends inside
-# a slice, fewer slices than K groups, and K splits.
+# a slice, fewer slices than K groups, and K splits; then K <= 64, whose tile a rule of its own picks
+# (64 x 64, 64 x 80, 64 x 96, 64 x 128 and 128 x 80, one to four slices).
 @pytest.mark.parametrize("beta", [0.0, -0.3])
 @pytest.mark.parametrize("ta,tb", [(0, 0), (0, 1), (1, 0), (1, 1)])
 @pytest.mark.parametrize("m,n,k,batch", [(63, 1, 40, 3), (65, 15, 95, 1), (95, 95, 31, 1), (361, 25, 361, 1), (90, 90, 9000, 1),
                                          (129, 143, 600, 1), (1891, 169, 200, 1), (777, 333, 111, 2), (3001, 145, 97, 1),
-                                         (2003, 801, 65, 1), (1000, 1001, 130, 1), (40, 2047, 77, 1)])
+                                         (2003, 801, 65, 1), (1000, 1001, 130, 1), (40, 2047, 77, 1),
+                                         (1, 1, 3, 1), (502, 1490, 15, 1), (2000, 300, 16, 1), (130, 90, 32, 2),
+                                         (1500, 701, 20, 1), (10001, 199, 10, 1),
+                                         (2500, 501, 33, 1), (901, 899, 64, 1)])
 def test_gemm_f64_tiles(ta, tb, m, n, k, batch, beta):
     from mpqc_amd.ccsd import gemm
     rng = np.random.default_rng(m + 2 * n + 3 * k)

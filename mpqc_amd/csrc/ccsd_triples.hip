@@ -536,11 +536,19 @@ void triples_sum(const TripleSumArgs& g, hipStream_t s) {
   }
 }
 
-// Up to this K = v + o the split-precision forms' (T) takes the FP64 sums too: planes cut the
-// products' time, which grows with K, but every ordering's W still goes through HBM.  FP64
-// sums against W from fp16 planes, ms: (o, v) = (20, 76) 17 : 38, (24, 110) 113 : 146,
-// (30, 130) 437 : 449, (20, 140) 157 : 163, (12, 190) 115 : 104, (40, 152) 1750 : 1360.
-constexpr long kSummedK = 160;
+// Whether the split-precision forms' (T) takes the FP64 sums too: planes cut the products' time,
+// which grows with K = v + o (in steps of 16), but every ordering's W still goes through HBM.  From
+// K = 145 to 160 the two are within 10 %, and planes are the faster where their blocks are long
+// (o > 20), tiles are filled (v >= 96) and rows of W start on 32 bytes (v a multiple of 4).  FP64 sums
+// against W from fp16 planes, ms, (o, v) = (20, 76) 17 : 38, (24, 110) 113 : 146, (40, 104) 439 : 492, (56, 88)
+// 747 : 829, (16, 144) 90 : 94, (20, 140) 157 : 163, (31, 129) 477 : 517, (50, 110) 1097 : 1165, (100, 60) 1450 :
+// 1786; (24, 136) 250 : 240, (32, 120) 398 : 380, (40, 120) 764 : 696, (60, 100) 1504 : 1441; (12, 190) 115 : 104,
+// (40, 152) 1750 : 1360.  bf16x6, with twice the plane products: (30, 130) 441 : 616, (60, 100) 1472 : 2048.
+bool summed_faster(long o, long v, GemmPrecision prec) {
+  const long K = v + o;
+  if (K <= 144) return true;
+  return K <= 160 && (prec == GemmPrecision::BF16X6 || !(o > 20 && v >= 96 && v % 4 == 0));
+}
 
 // acc[slot + block] = the block's run of partials[0..n), each summed in a fixed order
 constexpr int kSumBlocks = 32;
@@ -864,7 +872,7 @@ double CCSDContext::triples(double block_bytes, double* seconds) {
   MPQC_HIP_CHECK(hipEventCreate(&ev1));
   MPQC_HIP_CHECK(hipEventRecord(ev0, stream_));
   const std::vector<double> h =
-      split_mode() && V + o_ > kSummedK ? triples_orderings(block_bytes) : triples_summed(block_bytes);
+      split_mode() && !summed_faster(o_, V, prec_) ? triples_orderings(block_bytes) : triples_summed(block_bytes);
   MPQC_HIP_CHECK(hipEventRecord(ev1, stream_));
   MPQC_HIP_CHECK(hipEventSynchronize(ev1));
   float ms = 0.f;

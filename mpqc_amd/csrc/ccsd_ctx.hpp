@@ -395,7 +395,8 @@ class CCSDContext {
   double* levels_ws_ = nullptr;   // partial sums
   size_t levels_ws_n_ = 0;
   long levels_gen_ = -1;
-  static constexpr long kLevelMaxDoubles = 1L << 20;  // o^2 v^2
+  static constexpr long kLevelMaxDoubles = 1L << 20;      // o^2 v^2
+  static constexpr long kLevelMaxOoccDoubles = 1L << 23;  // o^4
   int levels_mode_ = 1;           // option "levels"
   bool levels_usable() const;
   void plan_levels();

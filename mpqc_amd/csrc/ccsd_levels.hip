@@ -182,11 +182,15 @@ __global__ __launch_bounds__(kLvThreads, 4) void level_kernel(const LevelOp* __r
 
 }  // namespace
 
-// Whether the scheduled form is the faster one (the table above).
+// Whether the scheduled form is the faster one: the table above; o^4 arrays too large for it, from
+// o = 54 or so ((o, v), op by op : by levels, us: (48, 21) 1029 : 1067, (56, 18) 1212 : 1320, (53, 8) 636 :
+// 525, (80, 6) 1329 : 1575, (100, 10) 3413 : 4225, (120, 4) 4466 : 5902); and one occupied orbital beside
+// many virtual ones, whose matrix-vector products are whole passes over HBM ((1, 150) 893 : 813, (1, 180)
+// 1330 : 1330, (1, 256) 3651 : 4103; (2, 256) 5380 : 4910).
 bool CCSDContext::levels_usable() const {
   const long O = o_, V = v_;
   return levels_mode_ && prec_ == GemmPrecision::F64 && !df_ && !direct_ && !tape_ && !kernel_timing_ &&
-         V * V * O * O <= kLevelMaxDoubles;
+         V * V * O * O <= kLevelMaxDoubles && O * O * O * O <= kLevelMaxOoccDoubles && (O > 1 || V <= 180);
 }
 
 void CCSDContext::plan_levels() {

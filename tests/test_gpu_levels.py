@@ -68,3 +68,21 @@ def test_levels_replan_on_new_integrals_and_options():
                 r = c.compute_residuals(a1, a2)
                 assert np.abs(r[0] - ref[0]).max() <= 1e-12 * np.abs(ref[0]).max()
                 assert np.abs(r[1] - ref[1]).max() <= 1e-12 * np.abs(ref[1]).max()
+
+
+# o^4 up to 2^23 and beyond it, where every op has a launch of its own with the option on too
+@pytest.mark.parametrize("no,nv,by_levels", [(53, 3, True), (54, 3, False)])
+def test_many_occupied_orbitals(no, nv, by_levels):
+    from mpqc_amd.ccsd import CCSD, Integrals
+    _, b, t1, t2 = _problem(no, nv)
+    ref = _oracle(b, t1, t2)
+    got = []
+    with CCSD(no, nv) as c:
+        c.set_integrals(Integrals(**b))
+        for levels in (1, 0):
+            c.set_option("levels", levels)
+            got.append(c.compute_residuals(t1, t2))
+    for r1, r2 in got:
+        assert np.abs(r1 - ref[0]).max() <= 1e-12 * max(np.abs(ref[0]).max(), 1e-3)
+        assert np.abs(r2 - ref[1]).max() <= 1e-12 * max(np.abs(ref[1]).max(), 1e-3)
+    assert np.array_equal(got[0][1], got[1][1]) != by_levels

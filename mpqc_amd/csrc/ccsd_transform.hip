@@ -80,7 +80,12 @@ void CCSDContext::transform_fock(int nbf, const double* fock, const double* Cact
 // and 9 GB at 144 functions and 30 + 114 orbitals; the tree takes 1.95e11 and 5 GB.)  p goes in
 // blocks and nu in slabs, so that Y1 to Y3 fit the scratch cache and calls after the first
 // allocate nothing.  Bound: the matrix cores (at
-// those sizes 15.0 -> 9.8 ms of kernels, 40 TFLOP/s, and 101-219 -> 10.6 ms for the call).
+// those sizes 15.0 -> 9.8 ms of kernels, 40 TFLOP/s, and 101-219 -> 10.6 ms for the call).  Up to
+// kFullTransform functions either form is a chain of short launches, 18 in the tree and 13 with all of
+// (pq|rs) and copies: the call with the blocks read back takes, us, all : tree, 205 : 240 at 15 functions,
+// 210 : 246 at 24, 300 : 352 at 48, 455 : 490 at 60, 558 : 541 at 64, 1030 : 980 at 80 (with all functions active).
+constexpr long kFullTransform = 60;
+
 void CCSDContext::transform_ao(int nbf, const double* eri, const double* fock, const double* c_occ,
                                const double* c_vir, int memspace) {
   if (nbf <= 0 || !eri || !fock || !c_occ || !c_vir) throw std::invalid_argument("transform_ao: null or empty input");
@@ -106,56 +111,81 @@ void CCSDContext::transform_ao(int nbf, const double* eri, const double* fock, c
     g.sA = sx; g.sC = so; g.batch = (int)batch;
     mpqc_hip::gemm(g, GemmPrecision::F64, ws_, stream_);
   };
-  // Y1 to Y3 take 2 GiB (every p block reads the AO integrals again, but a new context's first
-  // call pays 20 to 90 ms per GB for the allocation), 128 MiB of them for Y1
-  const long kSlab = 16L << 20, budget = (256L << 20) - kSlab;
-  struct Part { long nP, nR, nRQ, pb, slab; };  // p occupied, p virtual
-  Part part[2];
-  size_t words = 0;
-  for (int virt = 0; virt < 2; ++virt) {
-    Part& t = part[virt];
-    t.nP = virt ? V : O;
-    t.nR = virt ? V : nmo;  // r: all of Y2's last index (occupied first); only virtual ones for <ab|cd>
-    t.nRQ = virt ? V * V : std::max(O, V) * std::max(O, V);
-    const long per_p = n * n * t.nR + n * t.nRQ;
-    t.pb = ceil_div(t.nP, ceil_div(t.nP, std::max(1L, budget / per_p)));
-    t.slab = std::max(1L, std::min(n, kSlab / (n * n * t.pb)));
-    words = std::max<size_t>(words, (size_t)(t.slab * n * n * t.pb + t.pb * per_p));
-  }
-  ScratchBuf Y(scratch_, words);
-  for (int virt = 0; virt < 2; ++virt) {
-    const Part& t = part[virt];
-    const long nP = t.nP, c0 = virt ? O : 0, pb = t.pb, slab = t.slab;
-    double* const Y1 = Y.p;
-    double* const Y2 = Y1 + slab * n * n * pb;
-    double* const Y3 = Y2 + n * n * pb * t.nR;
-    for (long p0 = 0; p0 < nP; p0 += pb) {
-      const long np = std::min(pb, nP - p0);
-      double* Y2o = Y2;                                  // r occupied (p occupied only)
-      double* Y2v = Y2 + (virt ? 0 : n * n * np * O);    // r virtual
-      for (long m0 = 0; m0 < n; m0 += slab) {
-        const long ns = std::min(slab, n - m0);
-        quarter(x0 + m0 * n * n, ns * n * n, n * n * n, c0 + p0, np, Y1, 1, 0, 0);
-        if (!virt) quarter(Y1, n * np, n * np, 0, O, Y2o + m0 * n * np * O, ns, n * n * np, n * np * O);
-        quarter(Y1, n * np, n * np, O, V, Y2v + m0 * n * np * V, ns, n * n * np, n * np * V);
-      }
-      // the last two quarters of one choice of r and q, to the block(s) <pr|q.>
-      auto finish = [&](const double* y2, long R, long q0, long Q, double* dst_o, double* dst_v) {
-        quarter(y2, n * np * R, n * np * R, q0, Q, Y3, 1, 0, 0);
-        const long rows = np * R * Q;
-        if (dst_o) quarter(Y3, rows, rows, 0, O, dst_o + p0 * R * Q * O, 1, 0, 0);
-        quarter(Y3, rows, rows, O, V, dst_v + p0 * R * Q * V, 1, 0, 0);
-      };
-      if (virt) {
-        finish(Y2v, V, O, V, nullptr, Gabcd_);
-      } else {
-        finish(Y2o, O, 0, O, Gijkl_, Gijka_);
-        finish(Y2o, O, O, V, nullptr, Gijab_);
-        finish(Y2v, V, 0, O, nullptr, Giajb_);
-        finish(Y2v, V, O, V, nullptr, Giabc_);
+  auto full = [&] {
+    // all of (pq|rs), the leading index contracted four times, and the blocks as strided copies
+    ScratchBuf a(scratch_, (size_t)(n * n * n * nmo)), b(scratch_, (size_t)(n * n * nmo * nmo));
+    const double* x = x0;
+    long rows = n * n * n;
+    for (int k = 0; k < 4; ++k) {
+      double* const y = k % 2 ? b.p : a.p;
+      quarter(x, rows, rows, 0, nmo, y, 1, 0, 0);
+      x = y;
+      rows = rows / n * nmo;
+    }
+    struct Blk { double* dst; long P0, Q0, R0, S0, nP, nQ, nR, nS; };
+    const Blk blocks[] = {{Gijab_, 0, 0, O, O, O, O, V, V}, {Gijkl_, 0, 0, 0, 0, O, O, O, O},
+                          {Giajb_, 0, O, 0, O, O, V, O, V}, {Giabc_, 0, O, O, O, O, V, V, V},
+                          {Gijka_, 0, 0, 0, O, O, O, O, V}, {Gabcd_, O, O, O, O, V, V, V, V}};
+    const long m2 = nmo * nmo, s[4] = {m2 * nmo, nmo, m2, 1};
+    for (const Blk& q : blocks) {  // <PQ|RS>[a,b,c,d] = (P0+a, R0+c | Q0+b, S0+d)
+      const long ext[4] = {q.nP, q.nQ, q.nR, q.nS};
+      strided_copy(q.dst, ext, x, q.P0 * m2 * nmo + q.R0 * m2 + q.Q0 * nmo + q.S0, s, m2 * m2, stream_);
+    }
+  };
+  auto tree = [&] {
+    // Y1 to Y3 take 2 GiB (every p block reads the AO integrals again, but a new context's first
+    // call pays 20 to 90 ms per GB for the allocation), 128 MiB of them for Y1
+    const long kSlab = 16L << 20, budget = (256L << 20) - kSlab;
+    struct Part { long nP, nR, nRQ, pb, slab; };  // p occupied, p virtual
+    Part part[2];
+    size_t words = 0;
+    for (int virt = 0; virt < 2; ++virt) {
+      Part& t = part[virt];
+      t.nP = virt ? V : O;
+      t.nR = virt ? V : nmo;  // r: all of Y2's last index (occupied first); only virtual ones for <ab|cd>
+      t.nRQ = virt ? V * V : std::max(O, V) * std::max(O, V);
+      const long per_p = n * n * t.nR + n * t.nRQ;
+      t.pb = ceil_div(t.nP, ceil_div(t.nP, std::max(1L, budget / per_p)));
+      t.slab = std::max(1L, std::min(n, kSlab / (n * n * t.pb)));
+      words = std::max<size_t>(words, (size_t)(t.slab * n * n * t.pb + t.pb * per_p));
+    }
+    ScratchBuf Y(scratch_, words);
+    for (int virt = 0; virt < 2; ++virt) {
+      const Part& t = part[virt];
+      const long nP = t.nP, c0 = virt ? O : 0, pb = t.pb, slab = t.slab;
+      double* const Y1 = Y.p;
+      double* const Y2 = Y1 + slab * n * n * pb;
+      double* const Y3 = Y2 + n * n * pb * t.nR;
+      for (long p0 = 0; p0 < nP; p0 += pb) {
+        const long np = std::min(pb, nP - p0);
+        double* Y2o = Y2;                                  // r occupied (p occupied only)
+        double* Y2v = Y2 + (virt ? 0 : n * n * np * O);    // r virtual
+        for (long m0 = 0; m0 < n; m0 += slab) {
+          const long ns = std::min(slab, n - m0);
+          quarter(x0 + m0 * n * n, ns * n * n, n * n * n, c0 + p0, np, Y1, 1, 0, 0);
+          if (!virt) quarter(Y1, n * np, n * np, 0, O, Y2o + m0 * n * np * O, ns, n * n * np, n * np * O);
+          quarter(Y1, n * np, n * np, O, V, Y2v + m0 * n * np * V, ns, n * n * np, n * np * V);
+        }
+        // the last two quarters of one choice of r and q, to the block(s) <pr|q.>
+        auto finish = [&](const double* y2, long R, long q0, long Q, double* dst_o, double* dst_v) {
+          quarter(y2, n * np * R, n * np * R, q0, Q, Y3, 1, 0, 0);
+          const long rows = np * R * Q;
+          if (dst_o) quarter(Y3, rows, rows, 0, O, dst_o + p0 * R * Q * O, 1, 0, 0);
+          quarter(Y3, rows, rows, O, V, dst_v + p0 * R * Q * V, 1, 0, 0);
+        };
+        if (virt) {
+          finish(Y2v, V, O, V, nullptr, Gabcd_);
+        } else {
+          finish(Y2o, O, 0, O, Gijkl_, Gijka_);
+          finish(Y2o, O, O, V, nullptr, Gijab_);
+          finish(Y2v, V, 0, O, nullptr, Giajb_);
+          finish(Y2v, V, O, V, nullptr, Giabc_);
+        }
       }
     }
-  }
+  };
+  if (n <= kFullTransform) full();
+  else tree();
   check_launch("transform_ao");
   MPQC_HIP_CHECK(hipStreamSynchronize(stream_));
   have_ints_ |= 0x1f8u;

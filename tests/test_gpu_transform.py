@@ -128,11 +128,11 @@ def test_transform_df_matches_oracle_and_golden(reduced):
         assert _rel(c.get_integral("Gijab"), ref["Gijab"]) < 1e-12
 
 
-@pytest.mark.parametrize("nbf,o,v", [(15, 9, 4), (96, 11, 80), (120, 8, 100)])
+@pytest.mark.parametrize("nbf,o,v", [(15, 9, 4), (60, 13, 41), (61, 40, 12), (96, 11, 80), (120, 8, 100)])
 def test_transform_ao_blocks_and_slabs(nbf, o, v):
-    """More occupied than virtual orbitals; several slabs of the first AO index; several blocks of
-    the first orbital.  AO "integrals" without any permutational symmetry, device buffers,
-    against torch in float64 (the file's bar)."""
+    """All of (pq|rs) up to 60 functions, the tree beyond; more occupied than virtual orbitals in both;
+    several slabs of the first AO index; several blocks of the first orbital.  AO "integrals" without
+    any permutational symmetry, device buffers, against torch in float64 (the file's bar)."""
     import ctypes
     import torch
     from mpqc_amd import _lib as L

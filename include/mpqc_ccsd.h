@@ -329,7 +329,10 @@ int mpqc_ccsd_batch_time_stages(mpqc_ccsd_batch* b, int reps);
 int mpqc_ccsd_batch_get_stages(mpqc_ccsd_batch* b, int max_rows, int* n_rows, char* tags, int* kinds,
                                int* bm, int64_t* target, double* ms, double* flops);
 
-/* Device-pointer kernel entry points (stream may be NULL for the null stream). */
+/* Device-pointer kernel entry points (stream may be NULL for the null stream).  Split-K partial
+ * sums live in one workspace per GPU that the library allocates and keeps: calls that use it take
+ * turns on the device, whatever streams and threads they come from.  A call that is recorded into
+ * a graph is not ordered so; graphs that hold such calls must not run beside others. */
 int mpqc_ccsd_pp_ladder(int o, int v, const double* gabcd_dev, const double* tau_dev,
                         double* r2_dev, double alpha, double beta, int precision, void* stream);
 int mpqc_ccsd_gemm(int transa, int transb, int m, int n, int k, double alpha, const double* a,

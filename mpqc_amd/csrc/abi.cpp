@@ -94,29 +94,58 @@ int guarded_free(F&& f) {
 }
 
 // Split-K workspace for the context-free GEMM entry points: one per device,
-// grown on demand, kept until process exit.
+// grown on demand, kept until process exit.  Calls whose partial sums go there take turns: those on
+// one stream follow each other anyway; once a second stream has come up, each waits on the device
+// for the last one (an event, so callers of one stream pay nothing).
 struct FreeWorkspace {
   std::mutex m;
-  double* ptr[64] = {nullptr};
-  size_t bytes[64] = {0};
+  double* ptr = nullptr;
+  size_t bytes = 0;
+  hipStream_t last = nullptr;  // stream of the last call that may have left partial sums
+  bool used = false, shared = false;
+  hipEvent_t done = nullptr;   // end of that call (shared)
 };
-FreeWorkspace g_ws;
+FreeWorkspace g_ws[64];
 
-mpqc_hip::GemmWorkspace workspace_for_current_device(size_t want) {
+// gemm() on `want` bytes of the current device's workspace.  The plan is made for these bytes, not for
+// what an earlier call may have left, so that a call's result does not depend on the calls before it.
+void gemm_on_workspace(const mpqc_hip::GemmDesc& d, mpqc_hip::GemmPrecision prec, size_t want, hipStream_t stream) {
   int dev = 0;
   MPQC_HIP_CHECK(hipGetDevice(&dev));
   if (dev < 0 || dev >= 64) throw std::runtime_error("device index out of range");
-  std::lock_guard<std::mutex> lk(g_ws.m);
-  if (g_ws.bytes[dev] < want) {
-    if (g_ws.ptr[dev]) MPQC_HIP_CHECK(hipFree(g_ws.ptr[dev]));
-    g_ws.ptr[dev] = nullptr;
-    g_ws.bytes[dev] = 0;
+  FreeWorkspace& w = g_ws[dev];
+  std::lock_guard<std::mutex> lk(w.m);  // (also keeps the workspace from being regrown under a launch)
+  if (w.bytes < want) {
+    if (w.ptr) MPQC_HIP_CHECK(hipFree(w.ptr));
+    w.ptr = nullptr;
+    w.bytes = 0;
     void* p = nullptr;
     MPQC_HIP_CHECK(hipMalloc(&p, want));
-    g_ws.ptr[dev] = (double*)p;
-    g_ws.bytes[dev] = want;
+    w.ptr = (double*)p;
+    w.bytes = want;
   }
-  return {g_ws.ptr[dev], g_ws.bytes[dev]};
+  // (whether it leaves partial sums: planned, at the cost of half a microsecond, only where it matters)
+  const bool other = w.shared || (w.used && (stream != w.last || stream == hipStreamPerThread));
+  bool partials = other ? mpqc_hip::gemm_scratch_bytes(d, prec, want) > 0
+                        : prec != mpqc_hip::GemmPrecision::F64 || d.K >= 2 * mpqc_hip::kMinSplitK;
+  if (partials && other) {  // a call that a graph records is ordered by whoever launches the graph
+    hipStreamCaptureStatus st = hipStreamCaptureStatusNone;
+    if (hipStreamIsCapturing(stream, &st) != hipSuccess) (void)hipGetLastError();
+    partials = st == hipStreamCaptureStatusNone;
+  }
+  if (partials && w.shared) {
+    MPQC_HIP_CHECK(hipStreamWaitEvent(stream, w.done, 0));
+  } else if (partials && other) {
+    MPQC_HIP_CHECK(hipEventCreateWithFlags(&w.done, hipEventDisableTiming));
+    MPQC_HIP_CHECK(hipDeviceSynchronize());
+    w.shared = true;
+  }
+  mpqc_hip::gemm(d, prec, {w.ptr, want}, stream);
+  if (partials) {
+    if (w.shared) MPQC_HIP_CHECK(hipEventRecord(w.done, stream));
+    w.used = true;
+    w.last = stream;
+  }
 }
 
 // Scratch of the allocation-free GEMM entry: a fixed device array (one copy per
@@ -488,8 +517,7 @@ int mpqc_ccsd_gemm(int transa, int transb, int m, int n, int k, double alpha, co
                                                ldb, beta, c, ldc);
     d.sA = stride_a; d.sB = stride_b; d.sC = stride_c; d.batch = batch;
     const size_t want = std::max<size_t>((size_t)m * n * batch * 64 * sizeof(double), (size_t)64 << 20);
-    auto ws = workspace_for_current_device(std::min<size_t>(want, (size_t)1 << 30));
-    mpqc_hip::gemm(d, (mpqc_hip::GemmPrecision)precision, ws, (hipStream_t)stream);
+    gemm_on_workspace(d, (mpqc_hip::GemmPrecision)precision, std::min<size_t>(want, (size_t)1 << 30), (hipStream_t)stream);
   });
 }
 
@@ -528,8 +556,7 @@ int mpqc_ccsd_pp_ladder(int o, int v, const double* gabcd_dev, const double* tau
     // b("a,b,i,j") = tau("c,d,i,j") * Gabcd("a,b,c,d"): M = v^2, N = o^2, K = v^2
     mpqc_hip::GemmDesc d = mpqc_hip::make_gemm(false, false, (int)vv, (int)oo, (int)vv, alpha,
                                                gabcd_dev, vv, tau_dev, oo, beta, r2_dev, oo);
-    auto ws = workspace_for_current_device((size_t)1 << 20);
-    mpqc_hip::gemm(d, (mpqc_hip::GemmPrecision)precision, ws, (hipStream_t)stream);
+    gemm_on_workspace(d, (mpqc_hip::GemmPrecision)precision, (size_t)1 << 20, (hipStream_t)stream);
   });
 }
 

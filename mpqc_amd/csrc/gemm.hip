@@ -429,10 +429,10 @@ F64Plan plan_f64(const GemmDesc& d, size_t ws_bytes) {
     // be launched; the first, largest one stands for a shape that none can take)
     if (ti > 0 && (tiles + kXcdCount) * kThreads * c.kg >= kMaxThreads) continue;
     const double own = c.rb * c.cb * c.u * 256.0;  // products of a slice, per SIMD
-    // splits that give each CU up to three workgroups, at least 128 values of k long
+    // splits that give each CU up to three workgroups
     long last = 0;
     for (int want = 1; want <= 3; ++want) {
-      long ns = std::max<long>(1, std::min<long>(std::min<long>(512, d.K / 128), (long)want * kCUs / work));
+      long ns = std::max<long>(1, std::min<long>(std::min<long>(512, d.K / kMinSplitK), (long)want * kCUs / work));
       if (ns > 1) ns = std::max<long>(1, std::min<long>(ns, (long)(ws_bytes / slice_bytes)));
       const long chunk = ceil_div(slices, ns);
       ns = ceil_div(slices, chunk);
@@ -1285,7 +1285,7 @@ size_t gemm_scratch_bytes(const GemmDesc& d, GemmPrecision prec, size_t ws_bytes
   if (!g_thin_k_never && prec == GemmPrecision::F64 &&
       (thin_k_shape(d) || thin_n_shape(d) || small_batched_shape(d) || gemv_shape(d)))
     return 0;
-  if (prec == GemmPrecision::F64) return plan_f64(d, ws_bytes).scratch_bytes;
+  if (prec == GemmPrecision::F64) return d.K < 2 * kMinSplitK ? 0 : plan_f64(d, ws_bytes).scratch_bytes;
   const bool wide = wide_tiles(d, ws_bytes);
   return plan_splitk(d, wide ? 128 : 64, wide ? 128 : 64, ws_bytes).scratch_bytes;
 }

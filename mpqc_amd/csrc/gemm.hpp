@@ -39,6 +39,8 @@ struct GemmDesc {
   int batch = 1;
 };
 
+constexpr int kMinSplitK = 128;  // values of k of a K split of an FP64 contraction, at least
+
 // Workspace used for split-K partial sums (owned by the caller).
 struct GemmWorkspace {
   double* ptr = nullptr;

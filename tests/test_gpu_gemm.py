@@ -287,3 +287,61 @@ def test_gemm_f64_rows_past_a_two_group_grid():
     # each of k products and sums rounds once in either result
     bound = 2 * (k + 4) * 2.3e-16 * float(a.abs().max()) * float(b.abs().sum())
     assert float(c.abs().max()) <= bound
+
+
+# partial sums of calls on several streams share one workspace: each call's result is that of the
+# call alone, for short and long K splits and a split-precision form
+@pytest.mark.parametrize("prec", ["f64", "bf16x3"])
+def test_gemm_split_k_on_several_streams(prec):
+    from mpqc_amd.ccsd import gemm
+    gen = torch.Generator(device="cuda").manual_seed(2)
+    shapes = [(64, 48, 300), (90, 90, 9000), (33, 70, 2000), (128, 16, 480)]
+    ops = []
+    for m, n, k in shapes:
+        A = torch.randn(m, k, dtype=torch.float64, device="cuda", generator=gen)
+        B = torch.randn(k, n, dtype=torch.float64, device="cuda", generator=gen)
+        ops.append((m, n, k, A, B))
+
+    def run(op, out, stream):
+        m, n, k, A, B = op
+        gemm(0, 0, m, n, k, 1.0, A.data_ptr(), k, B.data_ptr(), n, 0.0, out.data_ptr(), n, precision=prec,
+             stream=stream.cuda_stream)
+
+    alone = []
+    for op in ops:
+        out = torch.empty(op[0], op[1], dtype=torch.float64, device="cuda")
+        run(op, out, torch.cuda.current_stream())
+        alone.append(out)
+    torch.cuda.synchronize()
+    streams = [torch.cuda.Stream() for _ in range(3)]
+    outs = [[torch.empty_like(alone[q % len(ops)]) for q in range(20)] for _ in streams]
+    torch.cuda.synchronize()
+    for q in range(20):
+        for s, stream in enumerate(streams):
+            run(ops[(q + s) % len(ops)], outs[s][(q + s) % len(ops) + len(ops) * (q // len(ops))], stream)
+    torch.cuda.synchronize()
+    for s in range(len(streams)):
+        for q in range(20):
+            k = (q + s) % len(ops)
+            assert torch.equal(outs[s][k + len(ops) * (q // len(ops))], alone[k]), (s, q)
+
+
+def test_ladder_plan_does_not_depend_on_earlier_calls():
+    """The ladder's K split is that of its own 1 MiB of workspace: here none, where 64 MiB would
+    split, before and after calls with a larger workspace."""
+    from mpqc_amd.ccsd import gemm, pp_ladder
+    o, v = 8, 40
+    gen = torch.Generator(device="cuda").manual_seed(3)
+    new = lambda *s: torch.randn(s, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    V, tau = new(v * v, v * v), new(v * v, o * o)
+    r = [torch.empty(v * v, o * o, dtype=torch.float64, device="cuda") for _ in range(3)]
+    torch.cuda.synchronize()
+    stream = torch.cuda.current_stream().cuda_stream
+    pp_ladder(V.data_ptr(), tau.data_ptr(), r[0].data_ptr(), o, v, stream=stream)
+    gemm(0, 0, v * v, o * o, v * v, 1.0, V.data_ptr(), v * v, tau.data_ptr(), o * o, 0.0, r[1].data_ptr(), o * o,
+         stream=stream)
+    pp_ladder(V.data_ptr(), tau.data_ptr(), r[2].data_ptr(), o, v, stream=stream)
+    torch.cuda.synchronize()
+    assert torch.equal(r[0], r[2])
+    assert not torch.equal(r[0], r[1])
+    assert float((r[0] - r[1]).abs().max()) <= 2 * 1604 * 2.3e-16 * float((V.abs() @ tau.abs()).max())

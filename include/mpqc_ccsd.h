@@ -162,7 +162,10 @@ const char* mpqc_ccsd_last_error(const mpqc_ccsd_ctx* ctx);
  * and FP32 residual is captured into a HIP graph on its second call and replayed; any option
  * change or new integrals re-capture; 0: eager launches), "levels" (1 default: the FP64 residual of the
  * standard method with o^2 v^2 <= 2^20 runs its small ops in a few launches of independent ones;
- * 0: one launch per op), "solve_restart" (1 default: solve()
+ * 0: one launch per op), "keep_scratch" (1 default: the context keeps the gigabytes of temporaries of
+ * mpqc_ccsd_transform_ao, _transform_df and _triples for its next calls, at most 4 GiB of them and 32 GiB
+ * over all contexts of the process; they go back when the context is destroyed and before an
+ * allocation of this library would fail; 0: each call frees them at its end, those kept at once), "solve_restart" (1 default: solve()
  * starts from the initial guess; 0: from the context's amplitudes; 2: from them projected onto
  * t2(a,b,i,j) = t2(b,a,j,i)).  Tuning keys that act on
  * every context of the process (measurement aids; the defaults are the measured best):

@@ -120,7 +120,7 @@ void gemm_on_workspace(const mpqc_hip::GemmDesc& d, mpqc_hip::GemmPrecision prec
     w.ptr = nullptr;
     w.bytes = 0;
     void* p = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&p, want));
+    MPQC_HIP_CHECK(mpqc_hip::device_malloc(&p, want));
     w.ptr = (double*)p;
     w.bytes = want;
   }

@@ -146,7 +146,7 @@ void CCSDBatch::plan() {
   if (ws_need > ws_n_) {
     if (ws_) MPQC_HIP_CHECK(hipFree(ws_));
     ws_ = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&ws_, std::max<size_t>(ws_need, 1) * sizeof(double)));
+    MPQC_HIP_CHECK(device_malloc((void**)&ws_, std::max<size_t>(ws_need, 1) * sizeof(double)));
     ws_n_ = std::max<size_t>(ws_need, 1);
   }
   for (Stage& s : stages_) build_plan(s);
@@ -221,9 +221,7 @@ bool CCSDBatch::side_by_side() {
     bytes += (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double);
   }
   if (50e-6 * size() > 0.6e-3 + flops / 30e12) return false;
-  size_t free = 0, total = 0;
-  MPQC_HIP_CHECK(hipMemGetInfo(&free, &total));
-  side_ = bytes < 0.5 * (double)free;
+  side_ = bytes < 0.5 * (double)device_available();
   return side_ == 1;
 }
 

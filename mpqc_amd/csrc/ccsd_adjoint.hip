@@ -61,7 +61,7 @@ int CCSDContext::adj_index(const double* p) {
   }
   if (!adj_[k]) {
     void* q = nullptr;
-    if (scratch_.allocate(&q, alloc_sizes_[k] * sizeof(double)) != hipSuccess) throw std::bad_alloc();
+    if (device_malloc(&q, alloc_sizes_[k] * sizeof(double)) != hipSuccess) throw std::bad_alloc();
     adj_[k] = (double*)q;
     adj_zero_[k] = 1;
   }
@@ -115,7 +115,7 @@ double* CCSDContext::adj_scratch(long n) {
   if (adj_scratch_n_ < n) {
     if (adj_scratch_) MPQC_HIP_CHECK(hipFree(adj_scratch_));
     adj_scratch_ = nullptr;
-    MPQC_HIP_CHECK(scratch_.allocate((void**)&adj_scratch_, n * sizeof(double)));
+    MPQC_HIP_CHECK(device_malloc((void**)&adj_scratch_, n * sizeof(double)));
     adj_scratch_n_ = n;
   }
   return adj_scratch_;
@@ -251,7 +251,7 @@ void CCSDContext::reverse_op(const TapeOp& op, bool integrals) {
           if (adj_ws_n_ < need) {
             if (adj_ws_) MPQC_HIP_CHECK(hipFree(adj_ws_));
             adj_ws_ = nullptr;
-            MPQC_HIP_CHECK(scratch_.allocate((void**)&adj_ws_, need * sizeof(double)));
+            MPQC_HIP_CHECK(device_malloc((void**)&adj_ws_, need * sizeof(double)));
             adj_ws_n_ = need;
           }
           d.C = adj_ws_;

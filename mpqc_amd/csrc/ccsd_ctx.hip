@@ -194,7 +194,7 @@ CCSDContext::~CCSDContext() { release(); }
 
 double* CCSDContext::alloc(size_t n) {
   void* p = nullptr;
-  if (scratch_.allocate(&p, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
+  if (device_malloc(&p, std::max<size_t>(n, 1) * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   allocations_.push_back((double*)p);
   alloc_sizes_.push_back(std::max<size_t>(n, 1));
   return (double*)p;
@@ -291,6 +291,9 @@ void CCSDContext::set_option(const std::string& key, double value) {
   } else if (key == "eom_n_guess") {
     if (value < 0 || value != (int)value) throw std::invalid_argument("eom_n_guess must be a non-negative integer");
     eom_n_guess_ = (int)value;
+  } else if (key == "keep_scratch") {  // 0: the temporaries of a call are freed at its end
+    if (value != 0.0 && value != 1.0) throw std::invalid_argument("keep_scratch must be 0 or 1");
+    scratch_.keep(value != 0.0);
   } else if (key == "triples_block_bytes") {
     if (!(value >= 1 << 20)) throw std::invalid_argument("triples_block_bytes must be at least 1 MiB");
     triples_block_bytes_ = value;
@@ -338,7 +341,7 @@ void CCSDContext::upload(double* dst, const double* src, const std::array<int, 4
     if (staging_n_ < (size_t)total) {
       if (staging_) MPQC_HIP_CHECK(hipFree(staging_));
       staging_ = nullptr;
-      MPQC_HIP_CHECK(scratch_.allocate((void**)&staging_, total * sizeof(double)));
+      MPQC_HIP_CHECK(device_malloc((void**)&staging_, total * sizeof(double)));
       staging_n_ = total;
     }
     MPQC_HIP_CHECK(hipMemcpyAsync(staging_, src, total * sizeof(double), hipMemcpyHostToDevice, stream_));
@@ -359,7 +362,7 @@ void CCSDContext::upload(double* dst, const double* src, const std::array<int, 4
   if (modeinfo_n_ < mi.size()) {
     if (modeinfo_) MPQC_HIP_CHECK(hipFree(modeinfo_));
     modeinfo_ = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&modeinfo_, mi.size() * sizeof(long)));
+    MPQC_HIP_CHECK(device_malloc((void**)&modeinfo_, mi.size() * sizeof(long)));
     modeinfo_n_ = mi.size();
   }
   MPQC_HIP_CHECK(hipMemcpyAsync(modeinfo_, mi.data(), mi.size() * sizeof(long), hipMemcpyHostToDevice, stream_));
@@ -397,7 +400,7 @@ void CCSDContext::download(double* dst, const double* src, const std::array<int,
   if (modeinfo_n_ < mi.size()) {
     if (modeinfo_) MPQC_HIP_CHECK(hipFree(modeinfo_));
     modeinfo_ = nullptr;
-    MPQC_HIP_CHECK(hipMalloc(&modeinfo_, mi.size() * sizeof(long)));
+    MPQC_HIP_CHECK(device_malloc((void**)&modeinfo_, mi.size() * sizeof(long)));
     modeinfo_n_ = mi.size();
   }
   MPQC_HIP_CHECK(hipMemcpyAsync(modeinfo_, mi.data(), mi.size() * sizeof(long), hipMemcpyHostToDevice, stream_));
@@ -406,7 +409,7 @@ void CCSDContext::download(double* dst, const double* src, const std::array<int,
     if (staging_n_ < (size_t)total) {
       if (staging_) MPQC_HIP_CHECK(hipFree(staging_));
       staging_ = nullptr;
-      MPQC_HIP_CHECK(scratch_.allocate((void**)&staging_, total * sizeof(double)));
+      MPQC_HIP_CHECK(device_malloc((void**)&staging_, total * sizeof(double)));
       staging_n_ = total;
     }
     ddst = staging_;
@@ -796,7 +799,7 @@ Planes CCSDContext::alloc_planes(long n, long row) {
   P.n = n;
   for (int q = 0; q < plane_count(plane_kind()); ++q) {
     void* ptr = nullptr;
-    MPQC_HIP_CHECK(scratch_.allocate(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)));
+    MPQC_HIP_CHECK(device_malloc(&ptr, std::max<long>(n, 8) * sizeof(uint16_t)));
     P.p[q] = (uint16_t*)ptr;
     plane_allocs_.push_back({P.p[q], (size_t)std::max<long>(n, 8)});
     if (P.row) MPQC_HIP_CHECK(hipMemsetAsync(ptr, 0, (size_t)n * sizeof(uint16_t), stream_));  // the gaps stay 0

@@ -309,7 +309,7 @@ class CCSDContext {
   std::vector<int64_t> occ_hm_, vir_hm_;
   std::vector<double*> allocations_;
   std::vector<size_t> alloc_sizes_;
-  ScratchCache scratch_;  // temporaries of transform_ao / transform_df and triples
+  ScratchCache scratch_;  // temporaries of transform_ao / transform_df and triples, kept between calls
 
   // density fitting (method "df"): three-index factors X(K,p,q) and their layouts
   bool df_ = false, reduced_abcd_ = true;

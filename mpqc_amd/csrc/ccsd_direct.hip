@@ -44,7 +44,7 @@ void CCSDContext::set_direct_ao(int nbf, const double* ao_eri, const double* c_o
   const long n4 = n * n * n * n;
   double* src = nullptr;
   if (!memspace) {
-    if (scratch_.allocate((void**)&src, (size_t)n4 * sizeof(double)) != hipSuccess) throw std::bad_alloc();
+    if (device_malloc((void**)&src, (size_t)n4 * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   }
   try {
     if (!memspace)

@@ -102,11 +102,7 @@ struct SlotPool {
   double* base = nullptr;
   std::vector<double*> free_;
   SlotPool(int nslots, long n) {
-    if (hipMalloc(&base, (size_t)nslots * n * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      base = nullptr;
-      throw std::bad_alloc();
-    }
+    if (device_malloc((void**)&base, (size_t)nslots * n * sizeof(double)) != hipSuccess) throw std::bad_alloc();
     for (int k = nslots - 1; k >= 0; --k) free_.push_back(base + (size_t)k * n);
   }
   ~SlotPool() {
@@ -132,7 +128,7 @@ void CCSDContext::ensure_abcd_from_factors() {
   const long Q = naux_, V = v_, vv = V * V;
   if (!Gabcd_) Gabcd_ = alloc((size_t)vv * vv);
   double* T = nullptr;
-  if (scratch_.allocate((void**)&T, (size_t)vv * vv * sizeof(double)) != hipSuccess) throw std::bad_alloc();
+  if (device_malloc((void**)&T, (size_t)vv * vv * sizeof(double)) != hipSuccess) throw std::bad_alloc();
   try {
     mpqc_hip::gemm(make_gemm(true, false, (int)vv, (int)vv, (int)Q, 1.0, Xab_, vv, Xab_, vv, 0.0, T, vv),
                    GemmPrecision::F64, ws_, stream_);
@@ -173,7 +169,6 @@ void CCSDContext::eom_apply_jt(const double* y, double* x) {
 }
 
 int CCSDContext::eom_ee(int n_roots, int max_iter, double convergence, int verbose, double* energies) {
-  scratch_.clear();  // (the vector pool may need the memory)
   if (n_roots < 1) throw std::invalid_argument("n_roots must be positive");
   if (max_iter < 1) throw std::invalid_argument("max_iter must be positive");
   if (!(convergence > 0.0)) throw std::invalid_argument("convergence must be positive");
@@ -356,10 +351,7 @@ int CCSDContext::eom_ee(int n_roots, int max_iter, double convergence, int verbo
     // A(ai,bj) = delta_ij F(a,b) - delta_ab F(i,j) + 2 <ij|ab> - <ia|jb>: the singles block of the
     // Jacobian at t = 0 (symmetric)
     double* A = nullptr;
-    if (hipMalloc(&A, (size_t)m * m * sizeof(double)) != hipSuccess) {
-      (void)hipGetLastError();
-      throw std::bad_alloc();
-    }
+    if (device_malloc((void**)&A, (size_t)m * m * sizeof(double)) != hipSuccess) throw std::bad_alloc();
     struct FreeA {
       double* p;
       ~FreeA() { (void)hipFree(p); }

@@ -469,9 +469,7 @@ bool CCSDContext::tape_pairs() {
   const double vv = (double)v_ * v_, oo = (double)o_ * o_;
   if (direct_ || vv * vv * oo < kPairWork || !pp_symmetric_usable()) return false;
   if (pv_sym_) return true;
-  size_t free = 0, total = 0;
-  MPQC_HIP_CHECK(hipMemGetInfo(&free, &total));
-  return (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double) < 0.5 * (double)free;
+  return (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double) < 0.5 * (double)device_available();
 }
 
 // tau^(c,d,i,j) (+)= sum_ab Gabcd(a,b,c,d) r2^(a,b,i,j), the ladder's adjoint in its amplitudes:

@@ -8,6 +8,7 @@
 //
 #include "gemm.hpp"
 #include "gemm_f64_tile.hpp"
+#include "scratch.hpp"
 
 #include <algorithm>
 
@@ -659,7 +660,7 @@ GroupedGemmPlan plan_grouped_gemm(const std::vector<GemmDesc>& probs, GemmPrecis
   }
   pl.ws_doubles = woff;
   pl.grid = (int)std::min<long>(pl.items, 4096);
-  MPQC_HIP_CHECK(hipMalloc(&pl.dev, host.size() * sizeof(GProblem)));
+  MPQC_HIP_CHECK(device_malloc(&pl.dev, host.size() * sizeof(GProblem)));
   MPQC_HIP_CHECK(hipMemcpyAsync(pl.dev, host.data(), host.size() * sizeof(GProblem),
                                 hipMemcpyHostToDevice, stream));
   MPQC_HIP_CHECK(hipStreamSynchronize(stream));

@@ -3,6 +3,7 @@
 // reads along the innermost output index.
 #include "tensor_ops.hpp"
 #include "permute.hpp"
+#include "scratch.hpp"
 
 #include <algorithm>
 #include <cmath>
@@ -623,7 +624,7 @@ GroupedPlan plan_grouped_tadd(const std::vector<GroupedTAddDesc>& probs, hipStre
     pl.items += (long)gr.x * gr.y * gr.z;
     pl.lds = std::max(pl.lds, perm_lds_bytes(host[q].g));
   }
-  MPQC_HIP_CHECK(hipMalloc(&pl.dev, host.size() * sizeof(GPerm)));
+  MPQC_HIP_CHECK(device_malloc(&pl.dev, host.size() * sizeof(GPerm)));
   MPQC_HIP_CHECK(hipMemcpyAsync(pl.dev, host.data(), host.size() * sizeof(GPerm), hipMemcpyHostToDevice, s));
   MPQC_HIP_CHECK(hipStreamSynchronize(s));
   return pl;
@@ -644,7 +645,7 @@ GroupedPlan plan_grouped_ew(const std::vector<GroupedEwDesc>& probs, hipStream_t
     host[q] = GEw{d.kind, d.out, d.a, d.b, d.n, d.o, d.v, pl.items};
     pl.items += ceil_div(d.n, kEwPerBlock);
   }
-  MPQC_HIP_CHECK(hipMalloc(&pl.dev, host.size() * sizeof(GEw)));
+  MPQC_HIP_CHECK(device_malloc(&pl.dev, host.size() * sizeof(GEw)));
   MPQC_HIP_CHECK(hipMemcpyAsync(pl.dev, host.data(), host.size() * sizeof(GEw), hipMemcpyHostToDevice, s));
   MPQC_HIP_CHECK(hipStreamSynchronize(s));
   return pl;

@@ -157,3 +157,26 @@ def test_transform_ao_blocks_and_slabs(nbf, o, v):
             c._check(c.lib.mpqc_ccsd_get_integral(c.ctx, L.INTEGRAL_IDS[name], ctypes.c_void_p(got.data_ptr()),
                                                   L.LAYOUT_DENSE, L.MEM_DEVICE))
             assert float((got - ref).abs().max() / ref.abs().max()) < 1e-12, name
+
+
+def test_scratch_goes_back_on_request():
+    """Option "keep_scratch": 0 gives the kept temporaries back and keeps none; the blocks are the same."""
+    import ctypes
+    import torch
+    from mpqc_amd import _lib as L
+    from mpqc_amd.ccsd import CCSD
+    nbf, o, v = 96, 11, 80
+    gen = torch.Generator(device="cuda").manual_seed(1)
+    new = lambda *s: torch.randn(s, dtype=torch.float64, device="cuda", generator=gen)  # noqa: E731
+    args = new(nbf, nbf, nbf, nbf), new(nbf, nbf), new(nbf, o), new(nbf, v)
+    with CCSD(o, v) as c:
+        got, free = [], []
+        for keep in (1, 1, 0):
+            c.set_option("keep_scratch", keep)
+            free.append(torch.cuda.mem_get_info()[0])
+            c._check(c.lib.mpqc_ccsd_transform_ao(c.ctx, nbf, *[ctypes.c_void_p(t.data_ptr()) for t in args], L.MEM_DEVICE))
+            free.append(torch.cuda.mem_get_info()[0])
+            got.append(c.get_integral("Gabcd"))
+    assert free[1] == free[2] == free[3]  # the second call allocates nothing
+    assert free[4] == free[5] > free[3]
+    assert np.array_equal(got[0], got[1]) and np.array_equal(got[0], got[2])

@@ -214,14 +214,15 @@ bool CCSDBatch::side_by_side() {
   if (side_ >= 0) return side_ == 1;
   side_ = 0;
   if (prec_ != GemmPrecision::F64) return false;
-  double flops = 0.0, bytes = 0.0;
+  double flops = 0.0, bytes = 0.0, later = 0.0;
   for (auto& m : mols_) {
     const double o = m->o_, v = m->v_, oo = o * o, vv = v * v;
     flops += 2.0 * oo * vv * vv + 14.0 * o * oo * v * vv;
     bytes += (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double);
+    if (!m->GiabcT_) later += o * v * vv * sizeof(double);  // (allocated by the first residual)
   }
   if (50e-6 * size() > 0.6e-3 + flops / 30e12) return false;
-  side_ = bytes < 0.5 * (double)device_available();
+  side_ = bytes < 0.5 * ((double)device_available() - later);
   return side_ == 1;
 }
 

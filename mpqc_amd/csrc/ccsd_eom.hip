@@ -209,6 +209,8 @@ int CCSDContext::eom_ee(int n_roots, int max_iter, double convergence, int verbo
       }
     }
   } restore{this, was_df, was_fov};
+  const int cap = std::max({nt * max_vector, n_guess, 3 * nt});
+  SlotPool pool(2 * cap + 3 * nt + 1, n);  // (before the recorded residual looks at the free memory)
   record_residual();  // the residual at the current amplitudes, recorded for the sweeps
 
   // preconditioner diagonals: FIJ(i,i), FAB(a,a) of the recorded residual
@@ -266,8 +268,6 @@ int CCSDContext::eom_ee(int n_roots, int max_iter, double convergence, int verbo
     ++eom_products_;
   };
 
-  const int cap = std::max({nt * max_vector, n_guess, 3 * nt});
-  SlotPool pool(2 * cap + 3 * nt + 1, n);
   double* scal = scalars_ + 16;
 
   // out[k] = <xs[k], y> over len elements

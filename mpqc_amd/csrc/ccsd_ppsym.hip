@@ -463,13 +463,18 @@ void CCSDContext::pp_ladder_symmetric(double* out) {
 }
 
 // Whether the ladder of an executed tape (FP64 or FP32 contractions) runs on pairs, forward and
-// in the sweep.  The first use packs V+ / V-, which only adjoint callers may not have done yet:
-// not where that would leave little of the device.
+// in the sweep.  The first use packs V+ / V-, which only adjoint callers may not have done yet: only
+// into half of the memory that is left when every array has its adjoint and Lambda its
+// vectors, so that a sweep which fits without the packed blocks fits with them.
 bool CCSDContext::tape_pairs() {
   const double vv = (double)v_ * v_, oo = (double)o_ * o_;
   if (direct_ || vv * vv * oo < kPairWork || !pp_symmetric_usable()) return false;
   if (pv_sym_) return true;
-  return (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double) < 0.5 * (double)device_available();
+  double later = 80.0 * oo * vv;
+  for (size_t k = 0; k < alloc_sizes_.size(); ++k)
+    if (k >= adj_.size() || !adj_[k]) later += (double)alloc_sizes_[k];
+  return (vv * (vv + 128.0) + 2.0 * (vv + 64.0) * oo) * sizeof(double) <
+         0.5 * ((double)device_available() - later * sizeof(double));
 }
 
 // tau^(c,d,i,j) (+)= sum_ab Gabcd(a,b,c,d) r2^(a,b,i,j), the ladder's adjoint in its amplitudes:

@@ -307,13 +307,20 @@ int mpqc_ccsd_get_integral_gradient(mpqc_ccsd_ctx* ctx, int which, double* out, 
 /* ---- batched residuals of many independent molecules ----
  * One context per molecule (o[k], v[k]; one tile per mode, so the tile layout is
  * the dense layout), residuals cc::compute_cs_ccsd_r1 + r2 (ccsd_r1_r2.h:70-293)
- * of all molecules in grouped launches captured in one hipGraph.  The reference
+ * of all molecules in grouped launches captured in one hipGraph, or, in FP64 batches of few or
+ * large molecules, every molecule's own residual on its own stream, all at once.  The reference
  * evaluates molecules one at a time; there is no batched counterpart. */
 typedef struct mpqc_ccsd_batch mpqc_ccsd_batch;
 int mpqc_ccsd_batch_create(int n_mol, const int* o, const int* v, int precision,
                            mpqc_ccsd_batch** out);
 int mpqc_ccsd_batch_destroy(mpqc_ccsd_batch* b);
 const char* mpqc_ccsd_batch_last_error(const mpqc_ccsd_batch* b);
+/* Options of a batch: "side_by_side" (-1 default: by molecule count, work and free memory, the last
+ * because the molecules' own residuals also hold packed blocks of about Gabcd's size; the two forms
+ * differ in the order of sums, within the rounding of FP64; 0: grouped launches; 1: side by side),
+ * "tile_edge" (64 or 128, default 64) and "split_target" (default 2048) of every grouped contraction,
+ * until mpqc_ccsd_batch_tune chooses them one by one. */
+int mpqc_ccsd_batch_set_option(mpqc_ccsd_batch* b, const char* key, double value);
 int mpqc_ccsd_batch_set_integral(mpqc_ccsd_batch* b, int mol, int which, const double* data,
                                  int layout, int memspace);
 int mpqc_ccsd_batch_set_amplitudes(mpqc_ccsd_batch* b, int mol, const double* t1, const double* t2,

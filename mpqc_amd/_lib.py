@@ -37,8 +37,8 @@ EXPORTS = [
     "mpqc_ccsd_get_kernel_times", "mpqc_ccsd_jacobian_transpose", "mpqc_ccsd_lambda_solve",
     "mpqc_ccsd_get_lambda", "mpqc_ccsd_energy_gradient", "mpqc_ccsd_get_integral_gradient",
     "mpqc_ccsd_batch_create", "mpqc_ccsd_batch_destroy", "mpqc_ccsd_batch_last_error",
-    "mpqc_ccsd_batch_set_integral", "mpqc_ccsd_batch_set_amplitudes", "mpqc_ccsd_batch_residual",
-    "mpqc_ccsd_batch_get_residuals", "mpqc_ccsd_batch_tune", "mpqc_ccsd_batch_time",
+    "mpqc_ccsd_batch_set_option", "mpqc_ccsd_batch_set_integral", "mpqc_ccsd_batch_set_amplitudes",
+    "mpqc_ccsd_batch_residual", "mpqc_ccsd_batch_get_residuals", "mpqc_ccsd_batch_tune", "mpqc_ccsd_batch_time",
     "mpqc_ccsd_batch_time_stages", "mpqc_ccsd_batch_get_stages",
 ]
 
@@ -104,6 +104,7 @@ def load():
         "mpqc_ccsd_batch_create": (I, [I, pI, pI, I, ctypes.POINTER(P)]),
         "mpqc_ccsd_batch_destroy": (I, [P]),
         "mpqc_ccsd_batch_last_error": (ctypes.c_char_p, [P]),
+        "mpqc_ccsd_batch_set_option": (I, [P, ctypes.c_char_p, D]),
         "mpqc_ccsd_batch_set_integral": (I, [P, I, I, P, I, I]),
         "mpqc_ccsd_batch_set_amplitudes": (I, [P, I, P, P, I, I]),
         "mpqc_ccsd_batch_residual": (I, [P]),

@@ -3,8 +3,10 @@
 Each molecule is evaluated with the reference's operator API
 (``cc::compute_cs_ccsd_r1`` + ``compute_cs_ccsd_r2``, ccsd_r1_r2.h:70-293);
 the batch runs all molecules' residuals as grouped launches captured in one
-hipGraph.  Tile edges and split-K targets of the grouped contractions come from
-the library's autotuner (``tune``).
+hipGraph, or, where that is the faster form (few or large molecules in FP64), each
+molecule's own residual on its own stream, all at once (option ``side_by_side``).
+Tile edges and split-K targets of the grouped contractions come from the library's
+autotuner (``tune``).
 """
 from __future__ import annotations
 
@@ -60,6 +62,11 @@ class CCSDBatch:
     def __len__(self):
         return len(self.o)
 
+    def set_option(self, key: str, value: float):
+        """``side_by_side`` (-1 the library's rule, 0 grouped launches, 1 side by side), ``tile_edge``
+        (64 or 128) and ``split_target`` of the grouped contractions."""
+        self._check(self.lib.mpqc_ccsd_batch_set_option(self.h, key.encode(), float(value)))
+
     def set_integrals(self, mol: int, blocks: Dict[str, np.ndarray]):
         for name, idx in L.INTEGRAL_IDS.items():
             a = np.ascontiguousarray(blocks[name], dtype=np.float64)
@@ -76,7 +83,7 @@ class CCSDBatch:
                                                             L.MEM_HOST))
 
     def residual(self):
-        """One residual per molecule (grouped launches, graph replay)."""
+        """One residual per molecule (grouped launches or side by side, by graph replay)."""
         self._check(self.lib.mpqc_ccsd_batch_residual(self.h))
 
     def get_residuals(self, mol: int):

@@ -420,6 +420,13 @@ const char* mpqc_ccsd_batch_last_error(const mpqc_ccsd_batch* b) {
   return b->err.c_str();
 }
 
+int mpqc_ccsd_batch_set_option(mpqc_ccsd_batch* b, const char* key, double value) {
+  return guarded_batch(b, [&](mpqc_hip::CCSDBatch& x) {
+    if (!key) throw std::invalid_argument("null option key");
+    x.set_option(key, value);
+  });
+}
+
 int mpqc_ccsd_batch_set_integral(mpqc_ccsd_batch* b, int mol, int which, const double* data,
                                  int layout, int memspace) {
   return guarded_batch(b, [&](mpqc_hip::CCSDBatch& x) {

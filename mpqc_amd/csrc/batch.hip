@@ -63,6 +63,25 @@ CCSDContext& CCSDBatch::mol(int k) {
   return *mols_[k];
 }
 
+void CCSDBatch::set_option(const std::string& key, double value) {
+  if (key == "side_by_side") {
+    if (value != -1.0 && value != 0.0 && value != 1.0) throw std::invalid_argument("side_by_side must be -1, 0 or 1");
+    route_ = (int)value;
+    side_ = -1;
+  } else if (key == "tile_edge") {
+    if (value != 64.0 && value != 128.0) throw std::invalid_argument("tile_edge must be 64 or 128");
+    defaults_.bm = (int)value;
+    planned_ = false;
+  } else if (key == "split_target") {
+    if (!(value >= 1.0 && value <= 65536.0) || value != (long)value)
+      throw std::invalid_argument("split_target must be an integer in [1, 65536]");
+    defaults_.target = (long)value;
+    planned_ = false;
+  } else {
+    throw std::invalid_argument("unknown batch option: " + key);
+  }
+}
+
 void CCSDBatch::release_graph() {
   if (exec_) (void)hipGraphExecDestroy(exec_);
   if (graph_) (void)hipGraphDestroy(graph_);
@@ -99,6 +118,8 @@ void CCSDBatch::plan() {
   size_t ws_need = 0;
   for (size_t i = 0; i < nops; ++i) {
     Stage st;
+    st.bm = defaults_.bm;
+    st.target = defaults_.target;
     const CCSDContext::TapeOp& op0 = tapes[0][i];
     st.kind = op0.kind;
     st.tag = op0.kind == CCSDContext::TapeOp::kGemm ? op0.tag
@@ -138,9 +159,11 @@ void CCSDBatch::plan() {
         }
       }
     }
-    if (st.kind == CCSDContext::TapeOp::kGemm)
+    if (st.kind == CCSDContext::TapeOp::kGemm) {
+      ws_need = std::max(ws_need, grouped_gemm_workspace(st.gemms, st.bm, st.target));
       for (const GroupedConfig& cf : grouped_candidates())
         ws_need = std::max(ws_need, grouped_gemm_workspace(st.gemms, cf.bm, cf.target));
+    }
     stages_.push_back(std::move(st));
   }
   if (ws_need > ws_n_) {
@@ -211,6 +234,7 @@ void CCSDBatch::ensure_planned() {
 // (20 of 12 to 16: 11.0 : 6.3).  The own forms also hold the ladder's packed blocks: not where
 // those would leave little of the device.
 bool CCSDBatch::side_by_side() {
+  if (route_ >= 0) return route_ == 1;
   if (side_ >= 0) return side_ == 1;
   side_ = 0;
   if (prec_ != GemmPrecision::F64) return false;

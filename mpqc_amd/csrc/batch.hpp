@@ -27,6 +27,9 @@ class CCSDBatch {
   ~CCSDBatch();
   int size() const { return (int)mols_.size(); }
   CCSDContext& mol(int k);
+  // "side_by_side": -1 the rule's choice, 0 grouped launches, 1 the molecules' own residuals;
+  // "tile_edge", "split_target": configuration of every grouped contraction (until tune())
+  void set_option(const std::string& key, double value);
 
   // one residual per molecule at its current amplitudes (graph replay)
   void residual();
@@ -49,6 +52,11 @@ class CCSDBatch {
   void time_stages(int reps);
 
  private:
+  struct GroupedDefaults {
+    int bm = 64;
+    long target = 2048;
+  } defaults_;
+  int route_ = -1;  // option "side_by_side"
   struct Stage {
     int kind = 0;
     std::string tag;

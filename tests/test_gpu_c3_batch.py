@@ -82,6 +82,7 @@ def test_256_hchains_batched_vs_single_and_oracle(prec):
     for gi, grp in enumerate(groups):
         print(f"{prec} group {gi}: {len(grp)} chains, o {sizes[grp[0]][0]}..{sizes[grp[-1]][0]}", flush=True)
         with CCSDBatch([sizes[k][0] for k in grp], [sizes[k][1] for k in grp], precision=prec) as B:
+            B.set_option("side_by_side", 0)  # (side by side is the single-molecule path)
             for j, k in enumerate(grp):
                 o, v = sizes[k]
                 b, _, _, t1, t2 = _chain_inputs(torch, k, o, v)

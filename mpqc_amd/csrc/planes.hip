@@ -137,7 +137,9 @@ __global__ __launch_bounds__(kPThreads) void split_write_kernel(PermGeom g, Spli
   const double sc = *o.scale;
   permute_block<SHAPE>(g, blockIdx.x, blockIdx.y, blockIdx.z, [&](long e, double v) {
     // row of e: the quotient's error, e 2^-52, is far below the half added (e < 2^50)
-    if (PAD) e += (long)(((double)e + 0.5) * o.inv_row) * o.pad;
+    // (the branch is always taken: without it the compiler forms all rows of a thread's elements
+    // side by side, and the registers that takes cost a sixth of the pass)
+    if (PAD && o.pad) e += (long)(((double)e + 0.5) * o.inv_row) * o.pad;
     const double x = v * sc;
     if (o.kind == (int)PlaneKind::F16x2) {
       const uint16_t h = f16_bits((float)x);

@@ -149,7 +149,8 @@ const char* mpqc_ccsd_last_error(const mpqc_ccsd_ctx* ctx);
 
 /* Numeric options: "fov_sign" (+1 reference F_VV as written, -1 exact CCSD for
  * non-Brillouin references), "precision" (MPQC_CCSD_PREC_*), "kernel_timing"
- * (1 = time every contraction with HIP events on the context stream),
+ * (1 = time every contraction with HIP events on the context stream; small residuals then run op by
+ * op instead of in levels, and eagerly, so that each phase can be timed),
  * "method" (0 standard, 1 df, 2 direct, 3 direct_df; ccsd.h:73, 94-99), "reduced_abcd_memory" (1 default:
  * the df method builds (ab|cd) lazily from Xab instead of reading Gabcd and
  * Giabc, ccsd.h:102,292), "df_block_bytes" (device memory for the lazily built
@@ -157,12 +158,16 @@ const char* mpqc_ccsd_last_error(const mpqc_ccsd_ctx* ctx);
  * the particle-particle ladder of ccsd_r1_r2.h:275 as two GEMMs over the symmetric and
  * antisymmetric (c,d) pair combinations, rows a<=b, with half the FLOPs, exact for any
  * amplitudes given Gabcd(b,a,d,c) = Gabcd(a,b,c,d), and W_oooo's Gijab tau term likewise given
- * Gijab(l,k,d,c) = Gijab(k,l,c,d); blocks without the symmetry and the adjoint's recorded
- * residual keep the full contractions; 0: the full contractions), "graph" (1 default: the FP64
+ * Gijab(l,k,d,c) = Gijab(k,l,c,d); blocks without the symmetry keep the full contractions.  The
+ * adjoint's products (mpqc_ccsd_jacobian_transpose, Lambda, EOM) run the ladder of the recorded residual and
+ * its transpose so too from o^2 v^4 = 3e8, and then hold packed blocks of about half of Gabcd's size,
+ * unless a solve of the context already packed them, as long as memory is ample: results can differ by the
+ * order of sums, within the rounding of FP64, with the free memory of the GPU; the integral
+ * gradient's dE/dGabcd uses the full contraction; 0: the full contractions everywhere), "graph" (1 default: the FP64
  * and FP32 residual is captured into a HIP graph on its second call and replayed; any option
  * change or new integrals re-capture; 0: eager launches), "levels" (1 default: the FP64 residual of the
- * standard method with o^2 v^2 <= 2^20 runs its small ops in a few launches of independent ones;
- * 0: one launch per op), "keep_scratch" (1 default: the context keeps the gigabytes of temporaries of
+ * standard method with o^2 v^2 <= 2^20 and o^4 <= 2^23 (and, for o = 1, v <= 180) runs its small ops in a
+ * few launches of independent ones; 0: one launch per op), "keep_scratch" (1 default: the context keeps the gigabytes of temporaries of
  * mpqc_ccsd_transform_ao, _transform_df and _triples for its next calls, at most 4 GiB of them and 32 GiB
  * over all contexts of the process; they go back when the context is destroyed and before an
  * allocation of this library would fail; 0: each call frees them at its end, those kept at once), "solve_restart" (1 default: solve()
